@@ -72,6 +72,8 @@ enum BoundCode : int {
 // `n` and sets `s` to the multiplicative sign (+1, -1, or 0 = "outside, reads
 // as zero").  In-range indices short-circuit (every bound maps them to
 // themselves with sign +1), so the integer modulo only runs on border taps.
+// The returned index is always in [0, n), also where the sign is 0, so that
+// an unguarded load through it stays inside the axis.
 // --------------------------------------------------------------------------
 template <typename I>
 __host__ __device__ inline I pos_mod(I a, I m) {
@@ -109,8 +111,11 @@ __host__ __device__ inline I fold(int b, I i, I n, int &s) {
       I p = 2 * (n + 1);
       I j = i < 0 ? n - i - 1 : i;
       j = j % p;
-      if (j % (n + 1) == n) s = 0;
-      else s = ((j / (n + 1)) & 1) ? -1 : 1;
+      if (j % (n + 1) == n) {   // between two reflections: reads as zero
+        s = 0;
+        return 0;
+      }
+      s = ((j / (n + 1)) & 1) ? -1 : 1;
       I k = (i == -1) ? I(0) : (i < 0 ? -i - 2 : i);
       k = pos_mod<I>(k, p);
       if (k == n) return n - 1;
