@@ -511,50 +511,69 @@ __global__ __launch_bounds__(BIN_NTH, 4) void bin_push(PPArgs<float> a, int nbx,
   }
 }
 
-// Host: the binned pass over the tiles listed in fb (count, scan, scatter,
-// one work-group per bin).  Returns false (nothing launched) when the
-// volume does not fit the packed sample positions or the scratch cannot be
-// allocated; the caller then runs its other second pass.
-template <int ORD, int MODE>
-static bool launch_binned(const PPArgs<float> &a, int ntx, int nty, int ntz, int64_t ntiles, const int *fb,
-                          hipStream_t st) {
-  using B = TileBox<ORD, !TileMeta<MODE>::gather>;
-  constexpr int TS = B::TX * B::TY * B::TZ;
+// Scratch of the binned pass: the tile list and the sort's arrays, in one
+// stream-ordered allocation.
+struct BinPlan {
+  int nbx, nby, nbz;
+  int64_t nbins, nsamp;
+  int *fb, *rest, *cnt, *start, *idx;   // fb: list (a count, then up to ntiles tile ids)
+};
+
+// Allocates a plan for ntiles tiles of TS samples and clears its counters.
+// False (nothing allocated) when the volume does not fit the packed sample
+// positions or the scratch cannot be had.
+static inline bool bin_plan(const PPArgs<float> &a, int64_t ntiles, int TS, BinPlan &p, hipStream_t st) {
   if (a.tZ > (1 << BIN_ZBITS) || a.tX * a.tY >= (int64_t(1) << 19)) return false;
-  const int nbx = (int)((a.sX + 2 * BIN_OFF + BIN_S - 1) / BIN_S);
-  const int nby = (int)((a.sY + 2 * BIN_OFF + BIN_S - 1) / BIN_S);
-  const int nbz = (int)((a.sZ + 2 * BIN_OFF + BIN_S - 1) / BIN_S);
-  const int64_t nbins = a.N * (int64_t)nbx * nby * nbz;
-  const int64_t nsamp = ntiles * TS;   // listed samples, at most
-  if (nbins >= (int64_t(1) << 31) || nsamp >= (int64_t(1) << 31)) return false;
+  p.nbx = (int)((a.sX + 2 * BIN_OFF + BIN_S - 1) / BIN_S);
+  p.nby = (int)((a.sY + 2 * BIN_OFF + BIN_S - 1) / BIN_S);
+  p.nbz = (int)((a.sZ + 2 * BIN_OFF + BIN_S - 1) / BIN_S);
+  p.nbins = a.N * (int64_t)p.nbx * p.nby * p.nbz;
+  p.nsamp = ntiles * TS;   // listed samples, at most
+  if (p.nbins >= (int64_t(1) << 31) || p.nsamp >= (int64_t(1) << 31)) return false;
   int *mem = nullptr;
-  if (scratch_alloc((void **)&mem, sizeof(int) * (size_t)(2 * nbins + 2 + nsamp), st) != hipSuccess) {
+  if (scratch_alloc((void **)&mem, sizeof(int) * (size_t)(2 * p.nbins + 3 + ntiles + p.nsamp), st) != hipSuccess) {
     (void)hipGetLastError();
     return false;
   }
-  // [rest count | cnt: nbins | start: nbins + 1 | idx: nsamp]
-  int *rest = mem, *cnt = mem + 1, *start = cnt + nbins, *idx = start + nbins + 1;
-  const int64_t gz = (nbins + NI_BLOCK - 1) / NI_BLOCK, gsamp = (nsamp + BIN_NTH - 1) / BIN_NTH;
-  hipLaunchKernelGGL(fill_zero<int>, dim3((unsigned)(gz < 65536 ? gz : 65536)), dim3(NI_BLOCK), 0, st, mem, nbins + 1);
-  const unsigned gs = (unsigned)(gsamp < 8192 ? gsamp : 8192);
-  hipLaunchKernelGGL((bin_sort<ORD, MODE, false>), dim3(gs), dim3(BIN_NTH), 0, st, a, ntx, nty, ntz, fb, nbx, nby,
-                     nbz, cnt, (const int *)start, idx, rest, (int)nsamp);
-  hipLaunchKernelGGL(bin_scan, dim3(1), dim3(1024), 0, st, fb, cnt, start, nbins);
-  hipLaunchKernelGGL((bin_sort<ORD, MODE, true>), dim3(gs), dim3(BIN_NTH), 0, st, a, ntx, nty, ntz, fb, nbx, nby,
-                     nbz, cnt, (const int *)start, idx, rest, (int)nsamp);
-  hipLaunchKernelGGL((bin_rest<ORD, MODE>), dim3(gs < 1024 ? gs : 1024), dim3(BIN_NTH), 0, st, a, ntx, nty, ntz, fb,
-                     (const int *)idx, (const int *)rest, (int)nsamp);
-  if constexpr (MODE == TM_PULL)
-    hipLaunchKernelGGL((bin_pull<ORD>), dim3((unsigned)nbins), dim3(BIN_NTH), 0, st, a, nbx, nby, nbz, fb,
-                       (const int *)start, (const int *)idx, nbins);
-  else if constexpr (MODE == TM_SGRAD)
-    hipLaunchKernelGGL((bin_grad<ORD>), dim3((unsigned)nbins), dim3(BIN_NTH), 0, st, a, nbx, nby, nbz, fb,
-                       (const int *)start, (const int *)idx, nbins);
-  else
-    hipLaunchKernelGGL((bin_push<ORD, MODE>), dim3((unsigned)nbins), dim3(BIN_NTH), 0, st, a, nbx, nby, nbz, fb,
-                       (const int *)start, (const int *)idx, nbins);
-  (void)hipFreeAsync(mem, st);
+  // [rest count | cnt: nbins | list count, tile ids: ntiles | start: nbins + 1 | idx: nsamp]
+  p.rest = mem;
+  p.cnt = mem + 1;
+  p.fb = p.cnt + p.nbins;
+  p.start = p.fb + 1 + ntiles;
+  p.idx = p.start + p.nbins + 1;
+  const int64_t gz = (p.nbins + 2 + NI_BLOCK - 1) / NI_BLOCK;
+  hipLaunchKernelGGL(fill_zero<int>, dim3((unsigned)(gz < 65536 ? gz : 65536)), dim3(NI_BLOCK), 0, st, mem,
+                     p.nbins + 2);
   return true;
+}
+
+// The binned pass over the tiles listed in the plan (count, scan, scatter,
+// one work-group per bin), then the plan's scratch is given back.  Without
+// extrapolation every in-bound sample's taps are within BIN_OFF voxels of
+// the source, so no sample is left to bin_rest.
+template <int ORD, int MODE>
+static void launch_binned(const PPArgs<float> &a, int ntx, int nty, int ntz, const BinPlan &p, hipStream_t st) {
+  const int64_t gsamp = (p.nsamp + BIN_NTH - 1) / BIN_NTH;
+  const unsigned gs = (unsigned)(gsamp < 8192 ? gsamp : 8192);
+  const int *fb = p.fb;
+  hipLaunchKernelGGL((bin_sort<ORD, MODE, false>), dim3(gs), dim3(BIN_NTH), 0, st, a, ntx, nty, ntz, fb, p.nbx, p.nby,
+                     p.nbz, p.cnt, (const int *)p.start, p.idx, p.rest, (int)p.nsamp);
+  hipLaunchKernelGGL(bin_scan, dim3(1), dim3(1024), 0, st, fb, p.cnt, p.start, p.nbins);
+  hipLaunchKernelGGL((bin_sort<ORD, MODE, true>), dim3(gs), dim3(BIN_NTH), 0, st, a, ntx, nty, ntz, fb, p.nbx, p.nby,
+                     p.nbz, p.cnt, (const int *)p.start, p.idx, p.rest, (int)p.nsamp);
+  if (a.extrap & 1)
+    hipLaunchKernelGGL((bin_rest<ORD, MODE>), dim3(gs < 1024 ? gs : 1024), dim3(BIN_NTH), 0, st, a, ntx, nty, ntz, fb,
+                       (const int *)p.idx, (const int *)p.rest, (int)p.nsamp);
+  if constexpr (MODE == TM_PULL)
+    hipLaunchKernelGGL((bin_pull<ORD>), dim3((unsigned)p.nbins), dim3(BIN_NTH), 0, st, a, p.nbx, p.nby, p.nbz, fb,
+                       (const int *)p.start, (const int *)p.idx, p.nbins);
+  else if constexpr (MODE == TM_SGRAD)
+    hipLaunchKernelGGL((bin_grad<ORD>), dim3((unsigned)p.nbins), dim3(BIN_NTH), 0, st, a, p.nbx, p.nby, p.nbz, fb,
+                       (const int *)p.start, (const int *)p.idx, p.nbins);
+  else
+    hipLaunchKernelGGL((bin_push<ORD, MODE>), dim3((unsigned)p.nbins), dim3(BIN_NTH), 0, st, a, p.nbx, p.nby, p.nbz,
+                       fb, (const int *)p.start, (const int *)p.idx, p.nbins);
+  (void)hipFreeAsync(p.rest, st);
 }
 
 }  // namespace ni_amd

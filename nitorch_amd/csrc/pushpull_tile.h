@@ -1,46 +1,38 @@
-// LDS-tiled pull / push / count / gradients for 3-D float fields (isotropic
-// order ORD).
+// LDS-tiled push / count for 3-D float fields (isotropic order ORD), and the
+// dispatch of every mode over the tiles, gathers and bins.
 //
 // One work-group owns a TX x TY x TZ tile of samples (grid points); each
 // thread owns R of them.  The work-group reduces the bounding box of the
 // first taps of its in-bound samples, and when the box (extended by the
-// ORD + 1 taps) fits in LDS:
-//  * gather modes (pull, gradients): stage the box of the source -- folded
-//            by the boundary condition and signed, so the taps need no
-//            folding -- in LDS, then read every tap from LDS;
-//  * push / count : accumulate the tile's splats into an LDS box of FP64
-//            values with FP64 LDS atomics (gfx950 runs ds_add_f64 at ~80% of
-//            the rate of its 64-bit integer atomics, and ~40x faster than
-//            ds_add_f32), then add the box to the output once, folded and
-//            signed, with one FP32 global atomic per non-zero box element.
-//            At orders >= 1 a thread's z-consecutive samples whose taps are
-//            z-consecutive too first sum their splats along z in registers
-//            (at most R = 4 or 2 FP32 terms a box element) and add one FP64
-//            atomic a position.  Every box element is a double sum of its splats
-//            (FP64 products at order 0; above, FP32 sums of at most R FP32
-//            products), so each output element keeps float's relative
-//            accuracy against the sum of its splats' magnitudes however
-//            small it is next to the tile's other values, and NaN / Inf
-//            values propagate as in the reference's float sums.
+// ORD + 1 taps) fits in LDS, it accumulates the tile's splats into an LDS
+// box of FP64 values with FP64 LDS atomics (gfx950 runs ds_add_f64 at ~80%
+// of the rate of its 64-bit integer atomics, and ~40x faster than
+// ds_add_f32), then adds the box to the output once, folded and signed, with
+// one FP32 global atomic per non-zero box element.  At orders >= 1 a
+// thread's z-consecutive samples whose taps are z-consecutive too first sum
+// their splats along z in registers (at most R = 4 or 2 FP32 terms a box
+// element) and add one FP64 atomic a position.  Every box element is a
+// double sum of its splats (FP64 products at order 0; above, FP32 sums of at
+// most R FP32 products), so each output element keeps float's relative
+// accuracy against the sum of its splats' magnitudes however small it is
+// next to the tile's other values, and NaN / Inf values propagate as in the
+// reference's float sums.
 // The box has fixed dimensions per order (every tap offset is then an
-// immediate of the LDS instruction); channels are staged NCC at a time.
+// immediate of the LDS instruction); channels are accumulated one at a time.
 // A tile whose box does not fit (scattered or far out-of-range
-// coordinates with extrapolation) is listed for a second pass.  Pull, push,
-// count and grid_grad: in calls of at least BIN_MIN_SAMPLES samples the
-// listed tiles' samples are sorted by first-tap bin and every bin runs with
-// a box of its own (pushpull_bin.h).  In smaller calls of pull, push and
-// count, and in the entry point that allocates nothing, tile_dyn cuts each
-// listed tile into sub-tiles with boxes sized to their own spread and runs
-// the direct per-sample routine pp_sample for a sub-tile that still does
-// not fit; tile_fallback runs pp_sample for the other gradient cases.  The
-// result never depends on the data's smoothness, only the speed does.
+// coordinates with extrapolation) is listed for a second pass: in calls of
+// at least BIN_MIN_SAMPLES samples the listed tiles' samples are sorted by
+// first-tap bin and every bin runs with a box of its own (pushpull_bin.h);
+// in smaller calls, and in the entry point that allocates nothing, tile_dyn
+// cuts each listed tile into sub-tiles with boxes sized to their own spread
+// and runs the direct per-sample routine pp_sample for a sub-tile that
+// still does not fit.  The result never depends on the data's smoothness,
+// only the speed does.
 //
 // Weights, the out-of-bound rule and the splat order of each sample are
 // those of pp_sample (nitorch/_C/src/impl/pushpull_common.cpp: OOB :926-974,
-// interpolate3d / splat3d :1176-1290, linear :1653-1858, nearest
-// :2314-2341); folding and signs follow bounds_common.h:28-219.  Gathers
-// sum the taps x-outer, z-inner (pp_sample: z-outer), which differs only by
-// rounding.
+// splat3d :1235-1290, linear :1653-1858, nearest :2314-2341); folding and
+// signs follow bounds_common.h:28-219.
 #pragma once
 #include <climits>
 
@@ -226,6 +218,14 @@ __device__ __forceinline__ int tl_taps(float x, float (&w)[ORD + 1], float (&g)[
     tl_weight<ORD, DERIV, 0>(x, lo, w, g);
     return lo;
   }
+}
+
+// First tap index of coordinate x (as tl_taps).
+template <int ORD>
+__device__ __forceinline__ int tl_first(float x) {
+  if constexpr (ORD == 0) return (int)roundf(x);
+  else if constexpr (ORD == 1) return (int)floorf(x);
+  else return (int)floorf(x - first_tap_offset<float>(ORD));
 }
 
 __device__ __forceinline__ int wave_min(int v) {
@@ -1274,67 +1274,84 @@ __global__ __launch_bounds__(DYN_NTH) void tile_dyn(PPArgs<float> a, int ntx, in
 }  // namespace ni_amd
 
 #include "pushpull_bin.h"   // the binned second pass (uses the helpers above)
+#include "pushpull_gather.h"
+#include "pushpull_gtile.h"
 
 namespace ni_amd {
 
-// tile_kernel, then tile_fallback on the tiles it listed as too scattered
-// (list in stream-ordered scratch; without it, tile_fallback repeats the
-// bounding-box test on every tile).
+// Channels from which the tiles of a large pull or grid_grad that are too
+// spread for a box of two channels are sorted into bins instead of staging
+// one channel at a time: with fewer, or in small calls, the sort costs more
+// than it saves (order 3, 181 x 217 x 181, a warp of 8 voxels RMS: 8 channels
+// 1.2 ms binned, 2.6 not; one channel 0.58 and 0.38).
+#define BIN_MIN_CHANNELS 3
+
+template <int ORD, int MODE>
+static void launch_gather_mode(const PPArgs<float> &a, hipStream_t st) {
+  if (a.C <= gather_channels<ORD, MODE>()) {
+    launch_gather<ORD, MODE>(a, st);
+    return;
+  }
+  if constexpr (ORD >= 2 && (MODE == TM_PULL || MODE == TM_SGRAD)) {
+    using B = TileBox<ORD, false>;
+    const int ntx = (int)((a.tX + B::TX - 1) / B::TX);
+    const int nty = (int)((a.tY + B::TY - 1) / B::TY);
+    const int ntz = (int)((a.tZ + B::TZ - 1) / B::TZ);
+    BinPlan p;
+    if (a.C >= BIN_MIN_CHANNELS && a.N * a.tX * a.tY * a.tZ >= BIN_MIN_SAMPLES &&
+        bin_plan(a, a.N * (int64_t)ntx * nty * ntz, B::TX * B::TY * B::TZ, p, st)) {
+      launch_gtile<ORD, MODE>(a, p.fb, st);
+      launch_binned<ORD, MODE>(a, ntx, nty, ntz, p, st);
+      return;
+    }
+  }
+  if constexpr (ORD > 0) launch_gtile<ORD, MODE>(a, nullptr, st);
+}
+
+// Push / count: tile_kernel, then the second pass on the tiles it listed as
+// too scattered (list in stream-ordered scratch or the caller's; without
+// either, tile_fallback repeats the bounding-box test on every tile).
 template <int ORD, int MODE>
 static void launch_tile(const PPArgs<float> &a, hipStream_t st) {
-  using B = TileBox<ORD, !TileMeta<MODE>::gather>;
-  const int ntx = (int)((a.tX + B::TX - 1) / B::TX);
-  const int nty = (int)((a.tY + B::TY - 1) / B::TY);
-  const int ntz = (int)((a.tZ + B::TZ - 1) / B::TZ);
-  const int64_t nb = a.N * (int64_t)ntx * nty * ntz;
-  const dim3 g((unsigned)nb), b(B::NTH);
-  int *fb = nullptr;
-  const bool own = a.scratch == nullptr;
-  if (!own) {
-    fb = a.scratch;   // the caller checked nb + 1 <= a.scratch_cap
-    hipLaunchKernelGGL(fill_zero<int>, dim3(1), dim3(NI_BLOCK), 0, st, fb, (int64_t)1);
-  } else if (scratch_alloc((void **)&fb, sizeof(int) * (size_t)(nb + 1), st) != hipSuccess) {
-    (void)hipGetLastError();
-    fb = nullptr;
+  if constexpr (TileMeta<MODE>::gather) {
+    launch_gather_mode<ORD, MODE>(a, st);
   } else {
-    hipLaunchKernelGGL(fill_zero<int>, dim3(1), dim3(NI_BLOCK), 0, st, fb, (int64_t)1);
-  }
-  if constexpr (MODE == TM_COUNT) {
-    hipLaunchKernelGGL((tile_kernel<ORD, MODE, 1>), g, b, 0, st, a, ntx, nty, ntz, nb, fb);
-  } else {
-    if (a.C == 1)
-      hipLaunchKernelGGL((tile_kernel<ORD, MODE, 1>), g, b, 0, st, a, ntx, nty, ntz, nb, fb);
-    else
-      hipLaunchKernelGGL((tile_kernel<ORD, MODE, B::MAX_NCC>), g, b, 0, st, a, ntx, nty, ntz, nb, fb);
-  }
-  if (fb) {
-    if constexpr (MODE == TM_PULL || MODE == TM_PUSH || MODE == TM_COUNT) {
-      // listed tiles: binned by first tap (when the call may allocate its
-      // bins and has at least BIN_MIN_SAMPLES samples: below that, the
-      // binned pass's six launches cost more than the sub-tile kernel's
-      // one), else sub-tiles with boxes sized to their spread
-      const bool big = a.N * a.tX * a.tY * a.tZ >= BIN_MIN_SAMPLES;
-      if (!own || !big || !launch_binned<ORD, MODE>(a, ntx, nty, ntz, nb, fb, st)) {
-        constexpr int nsub = (B::TX / DYN_TX) * (B::TY / DYN_TY) * (B::TZ / DYN_TZ);
-        const int64_t want = nb * nsub;
-        const unsigned gd = (unsigned)(want < 4096 ? want : 4096);
-        hipLaunchKernelGGL((tile_dyn<ORD, MODE>), dim3(gd), dim3(DYN_NTH), 0, st, a, ntx, nty, ntz, (const int *)fb);
-      }
+    using B = TileBox<ORD, true>;
+    const int ntx = (int)((a.tX + B::TX - 1) / B::TX);
+    const int nty = (int)((a.tY + B::TY - 1) / B::TY);
+    const int ntz = (int)((a.tZ + B::TZ - 1) / B::TZ);
+    const int64_t nb = a.N * (int64_t)ntx * nty * ntz;
+    const dim3 g((unsigned)nb), b(B::NTH);
+    int *fb = nullptr;
+    const bool own = a.scratch == nullptr;
+    // in calls of at least BIN_MIN_SAMPLES samples (below, the binned pass's
+    // launches cost more than the sub-tile kernel's one) that may allocate
+    BinPlan p;
+    const bool binned = own && a.N * a.tX * a.tY * a.tZ >= BIN_MIN_SAMPLES &&
+                        bin_plan(a, nb, B::TX * B::TY * B::TZ, p, st);
+    if (binned) {
+      fb = p.fb;
     } else {
-      // grid_grad's listed tiles take the binned pass in calls that may
-      // allocate and have BIN_MIN_SAMPLES samples; the other gradient modes,
-      // and grid_grad otherwise, run pp_sample over the listed tiles
-      bool done = false;
-      if constexpr (MODE == TM_SGRAD)
-        done = own && a.N * a.tX * a.tY * a.tZ >= BIN_MIN_SAMPLES && launch_binned<ORD, MODE>(a, ntx, nty, ntz, nb, fb, st);
-      if (!done) {
-        const unsigned gf = (unsigned)(nb < 2048 ? nb : 2048);
-        hipLaunchKernelGGL((tile_fallback<ORD, MODE>), dim3(gf), b, 0, st, a, ntx, nty, ntz, nb, (const int *)fb);
+      if (!own) {
+        fb = a.scratch;   // the caller checked nb + 1 <= a.scratch_cap
+      } else if (scratch_alloc((void **)&fb, sizeof(int) * (size_t)(nb + 1), st) != hipSuccess) {
+        (void)hipGetLastError();
+        fb = nullptr;
       }
+      if (fb) hipLaunchKernelGGL(fill_zero<int>, dim3(1), dim3(NI_BLOCK), 0, st, fb, (int64_t)1);
     }
-    if (own) (void)hipFreeAsync(fb, st);
-  } else {
-    hipLaunchKernelGGL((tile_fallback<ORD, MODE>), g, b, 0, st, a, ntx, nty, ntz, nb, (const int *)nullptr);
+    hipLaunchKernelGGL((tile_kernel<ORD, MODE, 1>), g, b, 0, st, a, ntx, nty, ntz, nb, fb);
+    if (binned) {
+      launch_binned<ORD, MODE>(a, ntx, nty, ntz, p, st);
+    } else if (fb) {
+      constexpr int nsub = (B::TX / DYN_TX) * (B::TY / DYN_TY) * (B::TZ / DYN_TZ);
+      const int64_t want = nb * nsub;
+      const unsigned gd = (unsigned)(want < 4096 ? want : 4096);
+      hipLaunchKernelGGL((tile_dyn<ORD, MODE>), dim3(gd), dim3(DYN_NTH), 0, st, a, ntx, nty, ntz, (const int *)fb);
+      if (own) (void)hipFreeAsync(fb, st);
+    } else {
+      hipLaunchKernelGGL((tile_fallback<ORD, MODE>), g, b, 0, st, a, ntx, nty, ntz, nb, (const int *)nullptr);
+    }
   }
 }
 

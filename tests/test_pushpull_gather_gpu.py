@@ -1,0 +1,83 @@
+"""GPU parity of the gathers (pull, grid_grad, the pull's grid gradient)
+against the FP64 oracle where their dispatch and their boxes change: channel
+counts on both sides of the cache / tile choice and of a partial channel
+chunk, tiles whose box needs four, two or one channel a stage or does not
+fit at all, lattices one off the 4 x 4 x 16 and 4 x 8 x 16 blocks, axes
+shorter than the taps, and sources whose z stride is not 1.
+
+Tolerances: 1e-5 norm-relative (float sums of at most (order + 1)^3 terms,
+(5 + 1)^3 ulps = 2.6e-5 at worst, a tenth of it in practice); order 0 exact.
+"""
+import numpy as np
+import pytest
+import torch
+
+from oracle import pushpull as O
+
+pytestmark = pytest.mark.gpu
+
+
+def T(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+def grid(rng, shape, source, kind):
+    g = np.stack(np.meshgrid(*[np.linspace(0, s - 1, n) for n, s in zip(shape, source)], indexing="ij"), -1)[None]
+    if kind == "stretch":       # neighbouring samples several voxels apart: wide boxes
+        g = (g - np.array(source) / 2) * 2.5 + np.array(source) / 2
+    elif kind == "scatter":     # no box holds a tile
+        g = rng.uniform(-3, np.array(source) + 2, g.shape)
+    g = g + rng.uniform(-0.6, 0.6, g.shape)
+    return g.astype(np.float32)
+
+
+def check(a, b, order, what):
+    a = a.detach().cpu().double().numpy()
+    if order == 0:
+        assert np.array_equal(a, b), what
+    assert np.abs(a - b).max() <= 1e-5 * max(np.abs(b).max(), 1e-30), what
+
+
+@pytest.mark.parametrize("order", [0, 1, 2, 3, 5, 7])
+@pytest.mark.parametrize("channels", [1, 2, 3, 4, 5])
+def test_gather_paths(order, channels):
+    from nitorch_amd import grid as G
+    rng = np.random.default_rng(100 * order + channels)
+    shapes = [((5, 9, 17), (5, 9, 17)), ((4, 8, 16), (37, 23, 41)), ((9, 7, 33), (40, 30, 50)), ((6, 5, 4), (3, 2, 4))]
+    for (shape, source), kind in zip(shapes, ("near", "stretch", "scatter", "near")):
+        g = grid(rng, shape, source, kind)
+        x = rng.standard_normal((1, channels) + source).astype(np.float32)
+        d = rng.standard_normal((1, channels) + shape).astype(np.float32)
+        g64, x64, d64 = (t.astype(np.float64) for t in (g, x, d))
+        for bound in ("dct2", "dst1", "dft", "zero"):
+            for extrap in (0, 1):
+                case = (kind, order, channels, bound, extrap)
+                # channels last: the source's z stride is the channel count
+                for xt in (T(x), T(np.moveaxis(x, 1, -1)).movedim(-1, 1)):
+                    out = G.grid_pull(xt, T(g), [bound], [order], extrap)
+                    check(out, O.grid_pull(x64, g64, bound, order, extrap, oob_f32=True), order, ("pull",) + case)
+                    if order == 0:
+                        continue
+                    out = G.grid_grad(xt, T(g), [bound], [order], extrap)
+                    check(out, O.grid_grad(x64, g64, bound, order, extrap, oob_f32=True), order, ("grad",) + case)
+                    gt = T(g).requires_grad_()
+                    out, = G.grid_pull_backward(T(d), xt, gt, [bound], [order], extrap)
+                    ref = O.grid_pull_backward(d64, x64, g64, bound, order, extrap, oob_f32=True)[1]
+                    check(out, ref, order, ("grid gradient",) + case)
+
+
+@pytest.mark.parametrize("order", [1, 2, 3])
+@pytest.mark.parametrize("channels", [1, 4])
+def test_outside_taps_are_not_read(order, channels):
+    """Under `zero`, a sample's taps outside the source read as zero whatever
+    the voxel they fold to holds; a NaN reaches only the samples whose own
+    taps touch it."""
+    from nitorch_amd import grid as G
+    rng = np.random.default_rng(order)
+    shape = (9, 10, 18)
+    g = grid(rng, shape, shape, "near")
+    x = rng.standard_normal((1, channels) + shape).astype(np.float32)
+    x[:, :, 0, 0, 0] = np.nan
+    out = G.grid_pull(T(x), T(g), ["zero"], [order], 1).cpu().numpy()
+    ref = O.grid_pull(x.astype(np.float64), g.astype(np.float64), "zero", order, 1, oob_f32=True)
+    assert np.isnan(ref).any() and np.array_equal(np.isnan(out), np.isnan(ref))
