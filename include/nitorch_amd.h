@@ -349,6 +349,26 @@ int ni_svf_mat3_mul(int32_t dtype, int64_t nvox, const void *a, const int64_t *a
 int ni_svf_grad_step(int32_t dtype, int64_t nvox, const void *jac, const int64_t *jac_stride, const void *p,
                      const int64_t *p_stride, const void *g0, const int64_t *g0_stride, void *out, void *stream);
 
+/* One linear squaring of a velocity field u = scale v, v [N, *shape, 3]
+ * (contiguous, every axis >= 2), in one pass: v_out = u + u o (id + u) (+ id
+ * with add_identity), the pull folded by `bound` (nitorch/spatial/_svf.py:
+ * 85-94).  With jac_out: the composed Jacobian ((I + D u) o (id + u)) jac, D
+ * periodic central differences (:449-478); jac NULL: the identity.  With
+ * g_out: gscale (g + det(jac) jac^T (g o (id + u))) (:271-279).  Outputs that
+ * are NULL are not computed; v_out and g_out differ from v and g, jac_out may
+ * be jac.  Matrix fields are [N, *shape, 3, 3], or [9, N, *shape] with
+ * `planar`. */
+int ni_svf_step(int32_t dtype, int64_t N, const int64_t *shape, const int32_t *bound, const void *v, double scale,
+                const void *jac, const void *g, double gscale, void *v_out, void *jac_out, void *g_out, int32_t planar,
+                int32_t add_identity, void *stream);
+
+/* The start of the analytic backward (_svf.py:255-269): jac_out = I + D u
+ * under `bound`, u = scale v, and g_out = (2 I - jac_out)^-T rot^T g (rot
+ * NULL: the identity).  Matrix fields are [9, N, *shape]; jac_out may be rot,
+ * g_out differs from g. */
+int ni_svf_rotate(int32_t dtype, int64_t N, const int64_t *shape, const int32_t *bound, const void *v, double scale,
+                  const void *rot, const void *g, void *jac_out, void *g_out, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

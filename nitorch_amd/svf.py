@@ -13,19 +13,25 @@ the squarings (`anagrad=True`).
 
 Fields are channel-last like the reference: ([batch], *spatial, dim);
 Jacobians (..., dim, dim) with jac[..., i, j] = d psi_i / d x_j; symmetric
-Hessians stored sparse as (h00, h11, h22, h01, h02, h12).  3-D fields of
-3 x 3 matrices on the GPU are multiplied, and pushed forward through a
-squaring, by libnitorch_amd.so (`ni_svf_mat3_mul`, `ni_svf_grad_step`),
-reading transposed and channel-first views in place.
+Hessians stored sparse as (h00, h11, h22, h01, h02, h12).  Linear squarings
+of 3-D fields on the GPU run as one kernel each (`ni_svf_step`: velocity,
+composed Jacobian and pushed-forward gradient); at other orders, and with a
+Hessian, 3-D fields of 3 x 3 matrices are multiplied, and pushed forward
+through a squaring, by `ni_svf_mat3_mul` and `ni_svf_grad_step`, reading
+transposed and channel-first views in place.
 """
 import torch
 
 from . import _lib as L
 from . import spatial as SP
+from .grid import bound_to_nitorch, inter_to_nitorch, make_list
 
 L.register_signatures({
     "ni_svf_mat3_mul": [L._I32, L._I64, L._P, L._PI64, L._P, L._PI64, L._P, L._P],
     "ni_svf_grad_step": [L._I32, L._I64, L._P, L._PI64, L._P, L._PI64, L._P, L._PI64, L._P, L._P],
+    "ni_svf_step": [L._I32, L._I64, L._PI64, L._PI32, L._P, L.ctypes.c_double, L._P, L._P, L.ctypes.c_double, L._P,
+                    L._P, L._P, L._I32, L._I32, L._P],
+    "ni_svf_rotate": [L._I32, L._I64, L._PI64, L._PI32, L._P, L.ctypes.c_double, L._P, L._P, L._P, L._P, L._P],
 })
 
 
@@ -213,11 +219,69 @@ def _jhj(jac, hess):
                         out[..., 0, 1], out[..., 0, 2], out[..., 1, 2]], -1)
 
 
+# --------------------------------------------------------------------------
+# Linear squarings of 3-D fields, one launch each (`ni_svf_step`).
+# --------------------------------------------------------------------------
+def _fused(vel, interpolation, bound, *others):
+    """Bound codes if the fused squarings apply to the velocity (and the
+    contiguous fields `others` of its shape), else None: linear
+    interpolation, 3-D contiguous float32 / float64 GPU fields, at least two
+    voxels along each axis (one has no difference to take) and 32-bit offsets
+    within a volume."""
+    if not (vel.is_cuda and vel.dim() >= 4 and vel.shape[-1] == 3 and vel.dtype in (torch.float32, torch.float64)):
+        return None
+    shape = vel.shape[-4:-1]
+    if min(shape) < 2 or 3 * shape[0] * shape[1] * shape[2] >= 2 ** 31 - 1 or vel.numel() == 0:
+        return None
+    if any(int(o) != 1 for o in inter_to_nitorch(make_list(interpolation), "int")):
+        return None
+    if not all(t.is_contiguous() and t.shape == vel.shape and t.dtype == vel.dtype and t.device == vel.device
+               for t in (vel,) + others):
+        return None
+    codes = [int(b) for b in bound_to_nitorch(make_list(bound), "int")]
+    return (codes + codes[-1:] * 3)[:3]
+
+
+def _step(v, codes, v_out, scale=1., jac=None, jac_out=None, g=None, g_out=None, gscale=1., planar=False,
+          add_identity=False):
+    L.check(L.lib().ni_svf_step(
+        L.dtype_code(v.dtype), v.shape[:-4].numel(), L.i64arr(v.shape[-4:-1]), L.i32arr(codes), L.ptr(v), scale,
+        L.ptr(jac), L.ptr(g), gscale, L.ptr(v_out), L.ptr(jac_out), L.ptr(g_out), int(planar), int(add_identity),
+        L.stream_of(v)), "svf_step")
+
+
+class _Squarings(torch.autograd.Function):
+    """exp_forward without a gradient (a Function, so that transforms that
+    would need one of these kernels raise instead of passing them by)."""
+
+    @staticmethod
+    def forward(ctx, vel, scale, steps, codes, displacement, jacobian):
+        jac = torch.empty(vel.shape + (3,), dtype=vel.dtype, device=vel.device) if jacobian else None
+        v, out, spare = vel, torch.empty_like(vel), None
+        for k in range(steps):
+            _step(v, codes, out, 1. if k else scale, jac if k else None, jac,
+                  add_identity=not displacement and k + 1 == steps)
+            if k == 0 and steps > 1:
+                spare = torch.empty_like(vel)
+            v, out = out, (v if k else spare)
+        return (v, jac) if jacobian else v
+
+    @staticmethod
+    def backward(ctx, *grads):
+        raise NotImplementedError("the fused squarings have no autodiff backward")
+
+
 def exp_forward(vel, inverse=False, steps=8, interpolation="linear", bound="dft", displacement=False,
                 jacobian=False, _anagrad=False):
     """Scaling and squaring (nitorch/spatial/_svf.py:45-99): returns the
     transformation (or, with `displacement`, the displacement) exp(vel), and
     with `jacobian` its Jacobian accumulated over the squarings."""
+    codes = None
+    if steps > 0 and (_anagrad or not (vel.requires_grad and torch.is_grad_enabled())):
+        codes = _fused(vel, interpolation, bound)
+    if codes is not None:
+        scale = (-1. if inverse else 1.) / 2 ** steps
+        return _Squarings.apply(vel, scale, steps, codes, displacement, jacobian)
     vel = -vel if inverse else vel.clone()
     dim = vel.shape[-1]
     spatial = vel.shape[-1 - dim:-1]
@@ -235,6 +299,42 @@ def exp_forward(vel, inverse=False, steps=8, interpolation="linear", bound="dft"
     return (vel, jac) if jacobian else vel
 
 
+class _Backward(torch.autograd.Function):
+    """exp_backward of a gradient alone on the fused squarings.  Jacobians
+    stay in one planar buffer; the last pass of each sweep skips what nothing
+    reads any more (the velocity, then the Jacobian too)."""
+
+    @staticmethod
+    def forward(ctx, vel, grad, inverse, steps, codes, rotate):
+        bufs = [torch.empty_like(vel), torch.empty_like(vel)]
+        jac = torch.empty((9,) + vel.shape[:-1], dtype=vel.dtype, device=vel.device)
+        rotate = rotate and steps > 0
+        if rotate:
+            v = vel
+            for k in range(steps):
+                out = bufs[k % 2] if k + 1 < steps else None
+                _step(v, codes, out, 1. if k else 1. / 2 ** steps, jac if k else None, jac, planar=True)
+                v = out
+        sign = 1. if inverse else -1.
+        g, g_out = torch.empty_like(grad), torch.empty_like(grad)
+        L.check(L.lib().ni_svf_rotate(
+            L.dtype_code(vel.dtype), vel.shape[:-4].numel(), L.i64arr(vel.shape[-4:-1]), L.i32arr(codes), L.ptr(vel),
+            sign / 2 ** steps, L.ptr(jac if rotate else None), L.ptr(grad), L.ptr(jac), L.ptr(g), L.stream_of(vel)),
+            "svf_rotate")
+        v = vel
+        for k in range(steps):
+            last = k + 1 == steps
+            out = None if last else bufs[k % 2]
+            _step(v, codes, out, 1. if k else sign / 2 ** steps, jac, None if last else jac, g, g_out,
+                  -sign / 2 ** steps if last else 1., planar=True)
+            v, g, g_out = out, g_out, g
+        return g if steps else g.mul_(-sign)
+
+    @staticmethod
+    def backward(ctx, grad):
+        raise NotImplementedError("the analytic backward is not differentiated again")
+
+
 def exp_backward(vel, *gradhess, inverse=False, steps=8, interpolation="linear", bound="dft",
                  rotate_grad=False):
     """Gradient (and block-diagonal Hessian) with respect to the velocity
@@ -245,6 +345,11 @@ def exp_backward(vel, *gradhess, inverse=False, steps=8, interpolation="linear",
     grad, *rest = gradhess
     hess = rest[0] if rest else None
     opt = dict(bound=bound, interpolation=interpolation)
+    # (the initial Jacobian knows bounds by these names only)
+    known = isinstance(bound, str) and bound in ("dct2", "replicate", "dct1", "dst2", "dst1", "zero", "dft")
+    codes = _fused(vel, interpolation, bound, grad) if hess is None and known else None
+    if codes is not None:
+        return _Backward.apply(vel.detach(), grad.detach(), inverse, steps, codes, rotate_grad)
     dim = vel.shape[-1]
     shape = vel.shape[-dim - 1:-1]
     ident = SP.identity_grid(shape, dtype=vel.dtype, device=vel.device)
