@@ -418,7 +418,7 @@ static void rs_launch(const T *input, T *output, const RsArgs &a, bool adjoint, 
     const long long ns = (long long)a.N * a.C * a.ns[0] * a.ns[1] * a.ns[2];
     hipLaunchKernelGGL(rs_fill<T>, dim3(rs_blocks(ns)), dim3(RS_BLOCK), 0, st, output, ns, T(0));
     hipLaunchKernelGGL((resize_kernel<T, true>), dim3(rs_blocks(nthreads)), dim3(RS_BLOCK), 0, st, input, output, a);
-  } else if (!rs_separable<T>(input, output, a, st)) {
+  } else if (!rs_fused<T>(input, output, a, st) && !rs_separable<T>(input, output, a, st)) {
     hipLaunchKernelGGL((resize_kernel<T, false>), dim3(rs_blocks(nthreads)), dim3(RS_BLOCK), 0, st, input, output, a);
   }
 }

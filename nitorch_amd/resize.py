@@ -97,7 +97,7 @@ def _resize(input, output, factor, bound, interpolation, mode, do_adjoint, norma
             shape = [int(math.ceil(s / f)) for s, f in zip(input.shape[2:], f3)]
         else:
             shape = [int(math.floor(s * f)) for s, f in zip(input.shape[2:], f3)]
-        output = input.new_zeros([*input.shape[:2], *shape])
+        output = input.new_empty([*input.shape[:2], *shape])   # fully written by the call
     else:
         if output.shape[:2] != input.shape[:2] or output.dim() != input.dim():
             raise RuntimeError("resize(): expected input and output with the same batch and channel sizes")
@@ -185,7 +185,7 @@ def c_prolongation(input, factor=2., bound="dct2", shape=None, output=None):
         if not shape:
             factor = make_list(factor, 3)
             shape = [int((s * f) // 1) for s, f in zip(input.shape[2:], factor)]
-        output = input.new_zeros([*input.shape[:2], *shape])
+        output = input.new_empty([*input.shape[:2], *shape])   # fully written by the call
     return SV.fmg_prolongation(input, output, bound)
 
 
@@ -197,7 +197,7 @@ def c_restriction(input, factor=2., bound="dct2", shape=None, output=None):
         if not shape:
             factor = make_list(factor, 3)
             shape = [int(math.ceil(s / f)) for s, f in zip(input.shape[2:], factor)]
-        output = input.new_zeros([*input.shape[:2], *shape])
+        output = input.new_empty([*input.shape[:2], *shape])   # fully written by the call
     return SV.fmg_restriction(input, output, bound)
 
 

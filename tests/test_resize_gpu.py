@@ -206,3 +206,38 @@ def test_resize_view_at_odd_offset():
     a = RZ.resize(x, None, [0.5], ["dct2"], [3], ["edge"])
     b = RZ.resize(x.clone(), None, [0.5], ["dct2"], [3], ["edge"])
     assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dt", [torch.float64, torch.float32])
+@pytest.mark.parametrize("order", [0, 1, 3, 4, 7])
+def test_one_pass_edges_vs_oracle(dt, order):
+    """The one-pass resize where its tiles and lists change: outputs one off
+    the 4 / 16 x 8 x 32 tile, source axes across a bitmap word (32) and
+    shorter than the taps, taps that wrap to the far end, and factors on both
+    sides of what a tile can stage."""
+    from nitorch_amd import resize as RZ
+    tol = 1e-10 if dt == torch.float64 else 2e-5
+    rng = np.random.default_rng(order)
+    for shape, f in (((5, 9, 33), [1.0]), ((33, 17, 66), [0.5]), ((4, 8, 32), [2.1]), ((2, 3, 2), [4.0]),
+                     ((40, 70, 35), [0.13, 0.3, 0.9])):
+        x = rng.standard_normal((1, 2) + shape)
+        for bound in ("dft", "dct2", "dst1", "zero"):
+            for mode in (["edge"], ["center"]):
+                if min(RS.out_shape(shape, f, False)) < 2 and mode == ["center"]:
+                    continue
+                ref = RS.resize(x, f, bound, [order], [RS.mode_code(m) for m in mode])
+                out = RZ.resize(T(x, dt), None, f, [bound], [order], mode)
+                assert rel(out, ref) <= tol, (shape, f, bound, mode)
+    # enough output tiles for 16 planes a work-group
+    x = rng.standard_normal((1, 60, 18, 34, 70))
+    ref = RS.resize(x, [1.3], "dct2", [order], [RS.mode_code("edge")])
+    assert rel(RZ.resize(T(x, dt), None, [1.3], ["dct2"], [order], ["edge"]), ref) <= tol
+
+
+def test_one_pass_keeps_nan_local():
+    """A NaN reaches the outputs whose taps use its voxel, no others."""
+    from nitorch_amd import resize as RZ
+    x = np.random.default_rng(1).standard_normal((1, 1, 20, 24, 40))
+    x[0, 0, 9, 10, 11] = np.nan
+    out = RZ.resize(T(x), None, [0.5], ["dct2"], [3], ["edge"]).cpu().numpy()
+    assert np.array_equal(np.isnan(out), np.isnan(RS.resize(x, [0.5], "dct2", [3], [RS.mode_code("edge")])))
