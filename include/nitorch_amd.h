@@ -179,6 +179,11 @@ int ni_resize(int32_t dtype, int32_t dim, int64_t N, int64_t C, const int64_t *i
               int32_t do_adjoint, int32_t normalize, int32_t accumulate, const void *input, void *output,
               void *stream);
 
+/* Voxel coordinates A [x y z] + t of 3-D lattices (nitorch/spatial/_grid.py:
+ * 579-615): mat [nbatch, 3, 4] = [A | t], contiguous, on the device ->
+ * out [nbatch, *shape, 3]. */
+int ni_affine_grid(int32_t dtype, int64_t nbatch, const int64_t *shape, const void *mat, void *out, void *stream);
+
 /* ------------------------------------------------------------------------
  * Displacement-field solver (3-D).  Fields are [N, 3, *shape] and Hessians
  * [N, CC, *shape], contiguous, with CC in {1, 3, 6} (6 = h00 h11 h22 h01 h02

@@ -9,8 +9,11 @@ runs in the HIP backend (`nitorch_amd.grid`).
 """
 import torch
 
+from . import _lib as L
 from .grid import (GridPull, GridPush, GridCount, GridGrad, SplineCoeff, SplineCoeffND,
                    BoundType, InterpolationType, bound_to_nitorch, inter_to_nitorch)
+
+L.register_signatures({"ni_affine_grid": [L._I32, L._I64, L._PI64, L._P, L._P, L._P]})
 
 __all__ = ["grid_pull", "grid_push", "grid_count", "grid_grad",
            "spline_coeff", "spline_coeff_nd", "affine_grid", "resize", "resize_grid", "reslice",
@@ -240,6 +243,48 @@ def affine_grid(mat, shape, jitter=False):
     return _matvec(lin, ijk) + off
 
 
+class _AffineLattice(torch.autograd.Function):
+    """affine_grid of (..., 3, 4) float32 / float64 matrices on the GPU, in
+    one pass (a Function, so that transforms that would need to see through
+    the kernel raise instead of passing it by)."""
+
+    @staticmethod
+    def forward(ctx, mat, shape):
+        mat = mat.contiguous()
+        out = torch.empty(mat.shape[:-2] + tuple(shape) + (3,), dtype=mat.dtype, device=mat.device)
+        L.check(L.lib().ni_affine_grid(L.dtype_code(mat.dtype), mat.shape[:-2].numel(), L.i64arr(shape), L.ptr(mat),
+                                       L.ptr(out), L.stream_of(mat)), "affine_grid")
+        return out
+
+    @staticmethod
+    def backward(ctx, grad):
+        raise NotImplementedError("the lattice kernel has no autodiff backward")
+
+
+def _reslice_lattice(affine, affine_to, shape):
+    """Coordinates inv(affine) @ affine_to @ v of a target lattice's voxels.
+    On the GPU, the small matrix algebra runs on the host (its dozens of
+    launches would cost more than the image's) and the lattice in one
+    kernel."""
+    from .affine import affine_lmdiv
+    n = 1
+    for s in shape:
+        n *= s
+    if not (affine.is_cuda and affine.shape[-1] == 4 and affine.dtype in (torch.float32, torch.float64)
+            and affine.dtype == affine_to.dtype and affine_to.device == affine.device
+            and len(shape) == 3 and 0 < n < 2 ** 31
+            and not (torch.is_grad_enabled() and (affine.requires_grad or affine_to.requires_grad))):
+        return affine_grid(affine_lmdiv(affine, affine_to), shape)
+    if affine.shape == affine_to.shape:
+        a, b = torch.stack([affine, affine_to]).cpu()
+    else:
+        a, b = affine.cpu(), affine_to.cpu()
+    mat = affine_lmdiv(a, b)[..., :3, :]
+    if mat.shape[-2:] != (3, 4):
+        return affine_grid(affine_lmdiv(affine, affine_to), shape)
+    return _AffineLattice.apply(mat.contiguous().to(affine.device), shape)
+
+
 def _resize_lattice(image, factor, shape, anchor, dim):
     """The output shape and the per-axis `LatticeAxis` maps of a resize.
 
@@ -319,7 +364,6 @@ def reslice(image, affine, affine_to, shape_to=None, **kwargs):
     options (prefilter=True unless given).  Image (*batch, *channels,
     *spatial) with batch the affine's leading dimensions; returns
     (*batch, *channels, *shape_to)."""
-    from .affine import affine_lmdiv
     kwargs.setdefault("prefilter", True)
     image = torch.as_tensor(image)
     dtype = image.dtype if image.dtype.is_floating_point else torch.get_default_dtype()
@@ -332,7 +376,7 @@ def reslice(image, affine, affine_to, shape_to=None, **kwargs):
     shape_to = tuple(space if shape_to is None else shape_to)
     nbatch = int(torch.Size(lead).numel()) if lead else 0
     nchan = int(torch.Size(chans).numel()) if chans else 0
-    lattice = affine_grid(affine_lmdiv(affine, affine_to), shape_to)
+    lattice = _reslice_lattice(affine, affine_to, shape_to)
     if not nbatch:
         lattice = lattice[None]
     out = grid_pull(image.reshape((nbatch or 1, nchan or 1) + space), lattice, **kwargs)

@@ -241,3 +241,31 @@ def test_one_pass_keeps_nan_local():
     x[0, 0, 9, 10, 11] = np.nan
     out = RZ.resize(T(x), None, [0.5], ["dct2"], [3], ["edge"]).cpu().numpy()
     assert np.array_equal(np.isnan(out), np.isnan(RS.resize(x, [0.5], "dct2", [3], [RS.mode_code("edge")])))
+
+
+@pytest.mark.parametrize("dt,tol", [(torch.float64, 1e-13), (torch.float32, 1e-6)])
+def test_reslice_lattice(dt, tol):
+    """The lattice kernel against float64 coordinates: odd and single-voxel
+    lattices, batched and broadcast matrices; a singular matrix is refused and
+    a matrix with a gradient keeps the general path."""
+    from nitorch_amd import spatial as SP
+    from nitorch_amd.affine import affine_lmdiv
+    rng = np.random.default_rng(5)
+    for shape in ((1, 1, 1), (5, 7, 3), (17, 16, 65)):
+        for lead_a, lead_b in (((), ()), ((2,), (2,)), ((2,), ())):
+            def mats(lead):
+                m = np.zeros(lead + (4, 4))
+                m[..., :3, :] = rng.standard_normal(lead + (3, 4))
+                m[..., :3, :3] += 4 * np.eye(3)
+                m[..., 3, 3] = 1
+                return torch.from_numpy(m).to(dt)
+            a, b = mats(lead_a), mats(lead_b)
+            ref = SP.affine_grid(affine_lmdiv(a.double(), b.double()), shape)
+            out = SP._reslice_lattice(a.to(DEV), b.to(DEV), shape)
+            assert out.dtype == dt and out.shape == ref.shape
+            # float32: the 3 x 3 inverse rounds too (condition numbers below 10)
+            assert rel(out, ref.numpy()) <= 10 * tol
+    with pytest.raises(RuntimeError):
+        SP._reslice_lattice(torch.zeros(4, 4, dtype=dt, device=DEV), torch.eye(4, dtype=dt, device=DEV), (4, 4, 4))
+    a = torch.eye(4, dtype=dt, device=DEV).requires_grad_()
+    assert SP._reslice_lattice(torch.eye(4, dtype=dt, device=DEV), a, (4, 4, 4)).requires_grad
