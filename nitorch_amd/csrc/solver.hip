@@ -1135,9 +1135,9 @@ __global__ __launch_bounds__(SV_BLOCK) void precond_kernel(const T *__restrict__
 #define XF_MIN_OUT (1 << 16)   // transfers with at least this many outputs use the LDS-tiled kernel
 struct Xfer {
   int Xi, Yi, Zi, Xo, Yo, Zo;
-  double sc[3];
+  double sc[3], inv[3];   // input / output size of each axis, and its inverse
   int b[3];
-  float chscale[6];   // per-channel factors (FMG rescaling, at most 6 channels)
+  double chscale[6];   // per-channel factors (FMG rescaling, at most 6 channels)
   int scaled;         // 0: no per-channel factor (any number of channels)
 };
 
@@ -1170,7 +1170,7 @@ __global__ __launch_bounds__(SV_BLOCK) void transfer_kernel(const T *__restrict_
 #pragma unroll
     for (int k = 0; k < NT; ++k) {
       const double dd = xc - (double)(lo + k);
-      wt[d][k] = T(NT == 4 ? w_lin(dd / P.sc[d]) / P.sc[d] : w_quad(dd));
+      wt[d][k] = T(NT == 4 ? w_lin(dd * P.inv[d]) * P.inv[d] : w_quad(dd));
       off[d][k] = fold<int>(P.b[d], lo + k, sz[d], sg[d][k]) * st[d];
     }
   }
@@ -1281,7 +1281,7 @@ __global__ __launch_bounds__(SV_BLOCK) void transfer_tile(const T *__restrict__ 
 #pragma unroll
       for (int k = 0; k < NT; ++k) {
         const double dd = xc - (double)(lo + k);
-        wt[e][k] = T(NT == 4 ? w_lin(dd / P.sc[d]) / P.sc[d] : w_quad(dd));
+        wt[e][k] = T(NT == 4 ? w_lin(dd * P.inv[d]) * P.inv[d] : w_quad(dd));
       }
       *ob[e] = lo - lo0[d];
     }
@@ -1298,7 +1298,7 @@ __global__ __launch_bounds__(SV_BLOCK) void transfer_tile(const T *__restrict__ 
 #pragma unroll
     for (int k = 0; k < NT; ++k) {
       const double dd = xc - (double)(lo + k);
-      wx[k] = T(NT == 4 ? w_lin(dd / P.sc[0]) / P.sc[0] : w_quad(dd));
+      wx[k] = T(NT == 4 ? w_lin(dd * P.inv[0]) * P.inv[0] : w_quad(dd));
     }
     const T *bp = box + ((lo - lo0[0]) * BY + oy) * BZ + oz;
     T acc = T(0);
@@ -1527,16 +1527,17 @@ static void launch_relax(T *x, const T *g, const T *h, int CC, const Geo &G, con
 
 template <typename T>
 static void launch_transfer(const T *in, T *out, int N, int C, const int *si, const int *so,
-                            const int *bound, bool restrict_, const float *chscale, int accumulate,
+                            const int *bound, bool restrict_, const double *chscale, int accumulate,
                             hipStream_t st) {
   Xfer P;
   P.Xi = si[0]; P.Yi = si[1]; P.Zi = si[2];
   P.Xo = so[0]; P.Yo = so[1]; P.Zo = so[2];
   for (int d = 0; d < 3; ++d) {
     P.sc[d] = (double)si[d] / (double)so[d];
+    P.inv[d] = (double)so[d] / (double)si[d];
     P.b[d] = bound[d];
   }
-  for (int c = 0; c < 6; ++c) P.chscale[c] = (chscale && c < C) ? chscale[c] : 1.0f;
+  for (int c = 0; c < 6; ++c) P.chscale[c] = (chscale && c < C) ? chscale[c] : 1.0;
   P.scaled = chscale != nullptr;   // FMG callers pass C <= 6 factors
   const long long n = (long long)N * C * so[0] * so[1] * so[2];
   // the LDS-tiled kernel when every tile's input box fits its static box
@@ -1660,6 +1661,8 @@ static int run_pcg(T *x, const T *g, const T *h, int CC, const Geo &G, const Ste
   return 0;
 }
 
+#include "solver_coarse.h"
+
 // ------------------------------- FMG --------------------------------------
 struct Level {
   int sz[3];
@@ -1716,13 +1719,18 @@ static size_t cm_ws_elems(int N, int CC, const Level *L, int NL) {
     }
   return 2 * (size_t)N * 3 * mx + hs;
 }
-static size_t fmg_ws_bytes(int N, int CC, int has_w, const Level *L, int NL, int use_cg, size_t esz) {
+// bytes before the coarse levels' table
+static size_t fmg_table_offset(int N, int CC, int has_w, const Level *L, int NL, int use_cg, size_t esz) {
   size_t b = fmg_norms_offset(N, CC, has_w, L, NL, esz) + 2 * SV_SLOTS * sizeof(double);
   if (use_cg)
     b = align_up(b + 2 * pcg_field_elems(N, L[0].V) * esz, 256) + 4 * (size_t)N * SV_SLOTS * sizeof(double);
   else if (!has_w)
     b = align_up(b, 256) + cm_ws_elems(N, CC, L, NL) * esz;
-  return b;
+  return align_up(b, 256);
+}
+static size_t fmg_ws_bytes(int N, int CC, int has_w, const Level *L, int NL, int use_cg, size_t esz) {
+  return fmg_table_offset(N, CC, has_w, L, NL, use_cg, esz) +
+         (esz == 4 ? sizeof(CoarseArgs<float>) : sizeof(CoarseArgs<double>));
 }
 
 template <typename T>
@@ -1743,10 +1751,12 @@ struct FMG {
   T *cg_z, *cg_p;          // PCG smoother scratch (sized for level 0)
   double *cg_sc;
   double *norm_slots;      // 2 SV_SLOTS partials of ||r||^2, ||g||^2
+  int lc;                  // first level of coarse_kernel (NL: none)
+  CoarseArgs<T> *co_args;
   hipStream_t st;
 
-  void factors(int l, float f[3]) const {  // fine / coarse size ratio between l and l+1
-    for (int d = 0; d < 3; ++d) f[d] = (float)((double)L[l].sz[d] / (double)L[l + 1].sz[d]);
+  void factors(int l, double f[3]) const {  // fine / coarse size ratio between l and l+1
+    for (int d = 0; d < 3; ++d) f[d] = (double)L[l].sz[d] / (double)L[l + 1].sz[d];
   }
   // fmg_common.cpp:375-387: Gauss-Seidel, or PCG when use_cg
   void relax(int l) {
@@ -1768,13 +1778,13 @@ struct FMG {
       launch_relax<T>(x[l], gl, h[l], CC, G[l], S[l], N, P[l], nb_iter, st);
   }
   void restrict_field(const T *fine, T *coarse, int l) {   // level l -> l+1, displacement scaling
-    float f[3], cs[6] = {1, 1, 1, 1, 1, 1};
+    double f[3], cs[6] = {1, 1, 1, 1, 1, 1};
     factors(l, f);
     cs[0] = f[0]; cs[1] = f[1]; cs[2] = f[2];
     launch_transfer<T>(fine, coarse, N, 3, L[l].sz, L[l + 1].sz, bound, true, cs, 0, st);
   }
   void restrict_hess(const T *fine, T *coarse, int l) {
-    float f[3], cs[6] = {1, 1, 1, 1, 1, 1};
+    double f[3], cs[6] = {1, 1, 1, 1, 1, 1};
     factors(l, f);
     if (CC == 1) cs[0] = f[0] * f[0];
     else {
@@ -1784,7 +1794,7 @@ struct FMG {
     launch_transfer<T>(fine, coarse, N, CC, L[l].sz, L[l + 1].sz, bound, true, cs, 0, st);
   }
   void prolong(const T *coarse, T *fine, int l, int accumulate) {  // level l+1 -> l
-    float f[3], cs[6] = {1, 1, 1, 1, 1, 1};
+    double f[3], cs[6] = {1, 1, 1, 1, 1, 1};
     factors(l, f);
     cs[0] = f[0]; cs[1] = f[1]; cs[2] = f[2];
     launch_transfer<T>(coarse, fine, N, 3, L[l + 1].sz, L[l].sz, bound, false, cs, accumulate, st);
@@ -1792,21 +1802,75 @@ struct FMG {
   void residual(int l) {
     launch_reg<T>(x[l], h[l], CC, l == 0 ? g0 : g[l], r[l], G[l], S[l], N, 1, nullptr, st);
   }
+  // the pyramid's coarse levels, for coarse_kernel
+  void coarse_setup(void *dst) {
+    co_args = (CoarseArgs<T> *)dst;
+    if (lc >= NL) return;
+    CoarseArgs<T> a;
+    std::memset((void *)&a, 0, sizeof(a));
+    a.nl = NL - lc;
+    a.CC = CC;
+    a.nb_iter = nb_iter;
+    for (int d = 0; d < 3; ++d) a.b[d] = bound[d];
+    for (int l = lc; l < NL; ++l) {
+      CoarseLevel<T> &c = a.L[l - lc];
+      c.X = G[l].X; c.Y = G[l].Y; c.Z = G[l].Z;
+      c.h = h[l];
+      c.g = l == 0 ? const_cast<T *>(g0) : g[l];   // (the first level's is only read)
+      c.x = x[l];
+      c.S = S[l];
+      if (!use_cg) a.P[l - lc] = P[l];
+    }
+    hipLaunchKernelGGL(coarse_write<T>, dim3(1), dim3(1), 0, st, co_args, a);
+  }
+  // levels lc .. NL - 1: the full-multigrid start, or one V-cycle from lc
+  void coarse(int start, int nb_cycles, int zero) {
+    const dim3 grid((unsigned)N), block(CoarseCfg<T>::NTH);
+    if (use_cg)
+      hipLaunchKernelGGL((coarse_kernel<T, true>), grid, block, sizeof(CoarseLds<T, true>), st, co_args, start,
+                         nb_cycles, zero);
+    else
+      hipLaunchKernelGGL((coarse_kernel<T, false>), grid, block, sizeof(CoarseLds<T, false>), st, co_args, start,
+                         nb_cycles, zero);
+  }
   // one V-cycle from level `base` (fmg_common.cpp:202-220)
   void vcycle(int base) {
-    for (int l = base; l < NL - 1; ++l) {
+    if (base >= lc) return coarse(0, 0, 0);   // (base == lc: finer bases only otherwise)
+    const int down = lc < NL ? lc : NL - 1;   // first level that is not relaxed on the way down
+    for (int l = base; l < down; ++l) {
       relax(l);
       residual(l);
       restrict_field(r[l], g[l + 1], l);
-      launch_fill<T>(x[l + 1], (long long)N * 3 * L[l + 1].V, T(0), st);
+      if (l + 1 < lc) launch_fill<T>(x[l + 1], (long long)N * 3 * L[l + 1].V, T(0), st);
     }
-    relax(NL - 1);
-    for (int l = NL - 2; l >= base; --l) {
+    if (lc < NL) coarse(0, 0, 1);
+    else relax(NL - 1);
+    for (int l = down - 1; l >= base; --l) {
       prolong(x[l + 1], x[l], l, 1);
       relax(l);
     }
   }
 };
+
+// Whether coarse_kernel's LDS may be had on the current device (cached).
+template <typename T>
+static bool coarse_ready() {
+  static int cache[64] = {0};   // 1 yes, 2 no
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return false;
+  if (!cache[dev]) {
+    int v = 0;
+    const bool ok = hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) == hipSuccess &&
+                    (size_t)v >= std::max(sizeof(CoarseLds<T, false>), sizeof(CoarseLds<T, true>)) &&
+                    hipFuncSetAttribute((const void *)coarse_kernel<T, true>,
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, v) == hipSuccess &&
+                    hipFuncSetAttribute((const void *)coarse_kernel<T, false>,
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, v) == hipSuccess;
+    (void)hipGetLastError();
+    cache[dev] = ok ? 1 : 2;
+  }
+  return cache[dev] == 1;
+}
 
 template <typename T>
 static int fmg_setup(FMG<T> &F, int N, const int *sz, const T *hess, int CC, const T *weight, const T *grad,
@@ -1850,6 +1914,16 @@ static int fmg_setup(FMG<T> &F, int N, const int *sz, const T *hess, int CC, con
     for (int d = 0; d < 3; ++d) F.G[l].b[d] = bound[d];
     if (!use_cg) F.P[l] = make_plan(F.G[l], F.band);
   }
+  // the coarse levels that one launch handles
+  F.lc = F.NL;
+  size_t co_vox = 0;
+  if (!has_w && coarse_ready<T>())
+    while (F.lc > 0 && F.NL - F.lc < CO_LEVELS && F.L[F.lc - 1].V <= (size_t)CoarseCfg<T>::LIM &&
+           F.L[F.lc - 1].sz[0] + F.L[F.lc - 1].sz[1] + F.L[F.lc - 1].sz[2] <= CO_AXES &&
+           co_vox + F.L[F.lc - 1].V <= (size_t)CoarseCfg<T>::TAB &&
+           (use_cg || plan_classes(F.P[F.lc - 1]) <= CO_CLASSES))
+      co_vox += F.L[--F.lc].V;
+  F.coarse_setup((char *)ws + fmg_table_offset(N, F.CC, has_w, F.L, F.NL, use_cg, sizeof(T)));
   // class-major buffers (after the norm slots; sized by fmg_ws_bytes)
   for (int l = 0; l < 16; ++l) { F.cm[l] = 0; F.cm_h[l] = nullptr; }
   F.cm_x = F.cm_g = nullptr;
@@ -1887,8 +1961,14 @@ static int fmg_setup(FMG<T> &F, int N, const int *sz, const T *hess, int CC, con
 // fmg_common.cpp:187-222
 template <typename T>
 static void fmg_run(FMG<T> &F, int nb_cycles) {
-  F.relax(F.NL - 1);
-  for (int base = F.NL - 2; base >= 0; --base) {
+  int base = F.NL - 2;
+  if (F.lc < F.NL) {
+    F.coarse(1, nb_cycles, 0);
+    base = F.lc - 1;
+  } else {
+    F.relax(F.NL - 1);
+  }
+  for (; base >= 0; --base) {
     F.prolong(F.x[base + 1], F.x[base], base, 0);
     for (int c = 0; c < nb_cycles; ++c) F.vcycle(base);
   }

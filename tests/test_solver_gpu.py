@@ -292,3 +292,27 @@ def test_fmg_cg_vs_oracle(sv, dt):
                 ref = S.fmg_grid(h, g, bound=bound, nb_cycles=2, nb_iter=2, use_cg=True, **p)
                 tol = 2e-4 if dt == torch.float32 else 1e-9
                 assert rel(x, ref) <= tol, (shape, p, bound)
+
+
+@pytest.mark.parametrize("use_cg", [False, True])
+@pytest.mark.parametrize("case", [
+    # shape, N, CC, bound, penalty: levels of at most 1200 voxels (float) / 600
+    # (double) and X + Y + Z <= 64 run in one launch
+    ((12, 10, 10), 1, 6, "dft", 3, torch.float32),    # 1200: the whole solve in it
+    ((11, 11, 10), 2, 3, "dct2", 3, torch.float32),   # 1210: from the second level on
+    ((10, 10, 6), 1, 6, "dct2", 2, torch.float64),    # 600
+    ((67, 9, 5), 1, 1, "zero", 3, torch.float32),     # axes that sum to more than 64
+    ((21, 22, 17), 2, 6, "dst2", 3, torch.float64),   # 7854 -> 11 x 11 x 9 -> 6 x 6 x 5
+    ((3, 2, 5), 3, 3, "dct1", 1, torch.float32),      # no second level of any size
+    ((37, 30, 33), 1, 6, "replicate", 2, torch.float32),
+])
+def test_fmg_coarse_levels_vs_oracle(sv, case, use_cg):
+    shape, N, CC, bound, ip, dt = case
+    rng = np.random.default_rng(61)
+    p = PENS[ip]
+    g, h = system(rng, shape, CC=CC, N=N)
+    x = sv.fmg_grid_cf(T(h, dt), T(g, dt), None, pen_vec(p), (1, 1, 1), bound, 2, 2, use_cg=use_cg)
+    kw = dict(use_cg=True) if use_cg else dict(product_order=True)
+    ref = S.fmg_grid(h, g, bound=bound, nb_cycles=2, nb_iter=2, **kw, **p)
+    tol = (2e-4 if use_cg else 1e-4) if dt == torch.float32 else 1e-9
+    assert rel(x, ref) <= tol, case
