@@ -1,5 +1,6 @@
-// Binned second pass for the tiles that tile_kernel listed (pull / push /
-// count / grid_grad of strongly deformed grids).
+// Binned second pass for the tiles that gtile_kernel, tile_kernel or
+// scatter_kernel listed (pull / grid_grad, push / count of strongly deformed
+// grids).
 //
 // A tile of samples that a rotation, a zoom or a displacement with a large
 // Jacobian spreads over a wide region of the source has a bounding box far
@@ -120,7 +121,7 @@ template <int ORD, int MODE, bool SCATTER>
 __global__ __launch_bounds__(BIN_NTH) void bin_sort(PPArgs<float> a, int ntx, int nty, int ntz, const int *fb,
                                                     int nbx, int nby, int nbz, int *cnt, const int *start,
                                                     int *idx, int *rest, int nsamp) {
-  using B = TileBox<ORD, !TileMeta<MODE>::gather>;
+  using B = TileDims<ORD, MODE>;
   constexpr int TS = B::TX * B::TY * B::TZ;
   const int64_t total = (int64_t)fb[0] * TS;
   for (int64_t j = (int64_t)blockIdx.x * BIN_NTH + threadIdx.x; j < total; j += (int64_t)gridDim.x * BIN_NTH) {
@@ -146,7 +147,7 @@ __global__ __launch_bounds__(BIN_NTH) void bin_sort(PPArgs<float> a, int ntx, in
 template <int ORD, int MODE>
 __global__ __launch_bounds__(BIN_NTH) void bin_rest(PPArgs<float> a, int ntx, int nty, int ntz, const int *fb,
                                                     const int *idx, const int *rest, int nsamp) {
-  using B = TileBox<ORD, !TileMeta<MODE>::gather>;
+  using B = TileDims<ORD, MODE>;
   if (fb[0] == 0) return;
   const int nr = *rest;
   for (int r = blockIdx.x * BIN_NTH + threadIdx.x; r < nr; r += gridDim.x * BIN_NTH) {
@@ -517,6 +518,7 @@ struct BinPlan {
   int nbx, nby, nbz;
   int64_t nbins, nsamp;
   int *fb, *rest, *cnt, *start, *idx;   // fb: list (a count, then up to ntiles tile ids)
+  int *tiles;   // scatter_kernel's: a count, the number of tiles tile_kernel put in fb, then ids
 };
 
 // Allocates a plan for ntiles tiles of TS samples and clears its counters.
@@ -531,19 +533,21 @@ static inline bool bin_plan(const PPArgs<float> &a, int64_t ntiles, int TS, BinP
   p.nsamp = ntiles * TS;   // listed samples, at most
   if (p.nbins >= (int64_t(1) << 31) || p.nsamp >= (int64_t(1) << 31)) return false;
   int *mem = nullptr;
-  if (scratch_alloc((void **)&mem, sizeof(int) * (size_t)(2 * p.nbins + 3 + ntiles + p.nsamp), st) != hipSuccess) {
+  if (scratch_alloc((void **)&mem, sizeof(int) * (size_t)(2 * p.nbins + 5 + 2 * ntiles + p.nsamp), st) != hipSuccess) {
     (void)hipGetLastError();
     return false;
   }
-  // [rest count | cnt: nbins | list count, tile ids: ntiles | start: nbins + 1 | idx: nsamp]
+  // [rest count | cnt: nbins | list count, tile ids: ntiles | two counts, tile ids | start: nbins + 1 | idx: nsamp]
   p.rest = mem;
   p.cnt = mem + 1;
   p.fb = p.cnt + p.nbins;
-  p.start = p.fb + 1 + ntiles;
+  p.tiles = p.fb + 1 + ntiles;
+  p.start = p.tiles + 2 + ntiles;
   p.idx = p.start + p.nbins + 1;
-  const int64_t gz = (p.nbins + 2 + NI_BLOCK - 1) / NI_BLOCK;
+  const int64_t clear = p.nbins + 4 + ntiles;   // up to the second list's counts
+  const int64_t gz = (clear + NI_BLOCK - 1) / NI_BLOCK;
   hipLaunchKernelGGL(fill_zero<int>, dim3((unsigned)(gz < 65536 ? gz : 65536)), dim3(NI_BLOCK), 0, st, mem,
-                     p.nbins + 2);
+                     clear);
   return true;
 }
 
