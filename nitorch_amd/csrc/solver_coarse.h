@@ -340,6 +340,13 @@ struct Coarse {
       }
       const double pap = co_sum<NTH>(acc, m.red, flip);
       const T alpha = T(rz / (pap > 1e-12 ? pap : 1e-12));
+      if (it + 1 == a.nb_iter) {   // nothing reads the last residual and direction
+#pragma unroll
+        for (int k = 0; k < VPT; ++k)
+#pragma unroll
+          for (int c = 0; c < 3; ++c) xv[k][c] += alpha * p[k][c];
+        break;
+      }
       T z[VPT][3];
       acc = 0;
 #pragma unroll
