@@ -9,8 +9,9 @@
 // prolongation -- between barriers.  PCG: 160 x 192 x 160 (four such
 // levels), 2 cycles of 4 steps: 15.8 -> 11.4 ms a solve, of which 2.4 ms here (9
 // launches instead of about 1500).  Gauss-Seidel: 63 x 77 x 58, 2 cycles of 2
-// sweeps: 5.98 -> 5.37 ms, of which 2.4 ms here: a class step (about 1.2 us)
-// is one wavefront's 25 taps and their latency.
+// sweeps: 6.00 -> 5.16 ms, of which 2.2 ms here: a class step (about 1.1 us)
+// is one wavefront's 25 taps and their latency; reading what the next class
+// needs beside the solution before the barrier took it from 5.38 to 5.16.
 //
 // Formulas are those of the per-level kernels (pcg_*, relax_small,
 // reg_kernel, transfer_kernel); sums over voxels differ by their order.
@@ -138,19 +139,18 @@ __device__ __forceinline__ double co_sum(double v, double (*red)[NTH / 64], int 
   return s;
 }
 
-// (L u) of the voxel whose neighbour words start at nb, its own values in own.
+// (L u) of the voxel with neighbour words e, its own values in own.
 template <typename T>
-__device__ __forceinline__ void co_stencil(const Co4<T> *u, const unsigned *nb, bool signs, const StencilT<T> &S,
-                                           T (&own)[3], T (&out)[3]) {
+__device__ __forceinline__ void co_stencil(const Co4<T> *u, const unsigned (&e)[CO_WORDS], bool signs,
+                                           const StencilT<T> &S, T (&own)[3], T (&out)[3]) {
   T val[25][3];
 #pragma unroll
   for (int w = 0; w < CO_WORDS; ++w) {
-    const unsigned e = nb[w * CoarseCfg<T>::TAB];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const int q = 2 * w + h;
       if (q >= 25) break;
-      const unsigned f = h ? e >> 16 : e & 0xffffu;
+      const unsigned f = h ? e[w] >> 16 : e[w] & 0xffffu;
       const Co4<T> c = u[f >> 2];
       val[q][0] = c.x;
       val[q][1] = c.y;
@@ -166,6 +166,20 @@ __device__ __forceinline__ void co_stencil(const Co4<T> *u, const unsigned *nb, 
   for (int d = 0; d < 3; ++d) own[d] = val[0][d];
   auto at = [&](int c, int i, int j, int k) -> T { return val[co_place(i, j, k)][c]; };
   apply_L_core<T>(at, S, out);
+}
+
+// The same, the words read from nb.
+template <typename T>
+__device__ __forceinline__ void co_words(const unsigned *nb, unsigned (&e)[CO_WORDS]) {
+#pragma unroll
+  for (int w = 0; w < CO_WORDS; ++w) e[w] = nb[w * CoarseCfg<T>::TAB];
+}
+template <typename T>
+__device__ __forceinline__ void co_stencil(const Co4<T> *u, const unsigned *nb, bool signs, const StencilT<T> &S,
+                                           T (&own)[3], T (&out)[3]) {
+  unsigned e[CO_WORDS];
+  co_words<T>(nb, e);
+  co_stencil<T>(u, e, signs, S, own, out);
 }
 
 // Tables of the transfer from level I to level O (NT = 4: restriction, 3:
@@ -392,18 +406,42 @@ struct Coarse {
     publish(V, xv);
     const int base = first(l);
     const int *cls = m.cls[l];
-    for (int it = 0; it < a.nb_iter; ++it)
-      for (int col = 0; cls[col] < V; ++col) {
-        const int c0 = cls[col], c1 = cls[col + 1];
-        for (int k = c0 + (int)threadIdx.x; k < c1; k += NTH) {
-          const int v = m.mem[base + k];
-          T Lx[3], M[6], x[3];
-          co_stencil<T>(m.u, m.nb + base + v, signs, L.S, x, Lx);
+    // a class's first NTH members, one a thread: what does not depend on the
+    // solution is read before the barrier that the class waits for
+    unsigned e[CO_WORDS];
+    T g[3], M[6];
+    int v = -1;
+    auto fetch = [&](int k, int end) {
+      v = -1;
+      if (k >= end) return;
+      v = m.mem[base + k];
+      co_words<T>(m.nb + base + v, e);
 #pragma unroll
-          for (int c = 0; c < 6; ++c) M[c] = m.gh[(3 + c) * V + v];
-          gs_update<T>(Lx, L.S.diag, m.gh[v], m.gh[V + v], m.gh[2 * V + v], M, x[0], x[1], x[2]);
-          m.u[v] = Co4<T>{x[0], x[1], x[2], T(0)};
+      for (int c = 0; c < 3; ++c) g[c] = m.gh[c * V + v];
+#pragma unroll
+      for (int c = 0; c < 6; ++c) M[c] = m.gh[(3 + c) * V + v];
+    };
+    auto update = [&]() {
+      if (v < 0) return;
+      T Lx[3], x[3];
+      co_stencil<T>(m.u, e, signs, L.S, x, Lx);
+      gs_update<T>(Lx, L.S.diag, g[0], g[1], g[2], M, x[0], x[1], x[2]);
+      m.u[v] = Co4<T>{x[0], x[1], x[2], T(0)};
+    };
+    fetch(threadIdx.x, cls[1]);
+#pragma unroll 1
+    for (int it = 0; it < a.nb_iter; ++it)
+#pragma unroll 1
+      for (int col = 0; cls[col] < V; ++col) {
+        const int c1 = cls[col + 1];
+        update();
+#pragma unroll 1
+        for (int k = cls[col] + NTH + (int)threadIdx.x; k < c1; k += NTH) {
+          fetch(k, c1);
+          update();
         }
+        const int nx = c1 < V ? col + 1 : 0;
+        fetch(cls[nx] + (int)threadIdx.x, cls[nx + 1]);
         __syncthreads();
       }
 #pragma unroll
