@@ -129,6 +129,10 @@ __host__ __device__ inline I fold(int b, I i, I n, int &s) {
   }
 }
 
+// Whether positions first .. first + extent - 1 all lie in [0, n).  (`first`
+// may be any integer: `first + extent` could overflow.)
+__host__ __device__ inline bool axis_inside(int first, int extent, int n) { return first >= 0 && first <= n - extent; }
+
 // --------------------------------------------------------------------------
 // Spline evaluation.  For order O, the taps of a sample at coordinate x are
 // lo, lo+1, ..., lo+O with lo = floor(x - (O-1)/2) (round(x) for O = 0);

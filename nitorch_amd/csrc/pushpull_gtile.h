@@ -378,7 +378,7 @@ __global__ __launch_bounds__(256) void gtile_kernel(PPArgs<float> a, int ntx, in
   // (32-bit byte offsets of a plane position: 2 * 64 strides below 2^31)
   d.inner = !none && a.src_s[3] < (1 << 22) && a.src_s[4] < (1 << 22);
 #pragma unroll
-  for (int k = 0; k < 3; ++k) d.inner = d.inner && mn[k] >= 0 && mn[k] + d.e[k] <= sz[k];
+  for (int k = 0; k < 3; ++k) d.inner = d.inner && axis_inside(mn[k], d.e[k], sz[k]);
   d.base = mn[0] * (int)a.src_s[2] + mn[1] * (int)a.src_s[3] + mn[2] * (int)a.src_s[4];
   if (!d.inner)
     // folded offsets and signs of the box positions along each axis

@@ -1,0 +1,52 @@
+"""GPU checks of pulls at the limits of what their entry points take:
+extrapolated coordinates beyond the integer range or infinite, whose first
+taps saturate.
+
+Tolerance against the FP64 oracle: 1e-5 norm-relative, as the other gathers
+(float sums of at most (order + 1)^3 terms)."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import pushpull as O
+
+pytestmark = pytest.mark.gpu
+
+
+def T(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+def close(a, b):
+    a = a.detach().cpu().double().numpy()
+    return np.abs(a - b).max() <= 1e-5 * np.abs(b).max()
+
+
+@pytest.mark.parametrize("value", [3e9, 1e10, -1e10, np.inf, -np.inf])
+@pytest.mark.parametrize("axes", [(0,), (1,), (2,), (0, 1, 2)])
+@pytest.mark.parametrize("order", [1, 2, 3])
+def test_gather_beyond_the_integer_range(order, axes, value):
+    """Tiles of 4 x 8 x 16 samples: the first is ordinary, every sample of the
+    second lies at `value` along `axes`.  Under `zero` its finite coordinates
+    read as zero (weights stay finite up to order 3)."""
+    from nitorch_amd import grid as G
+    rng = np.random.default_rng(order)
+    shape, source = (4, 8, 32), (9, 10, 40)
+    g = np.stack(np.meshgrid(*[np.arange(n, dtype=np.float64) + 2 for n in shape], indexing="ij"), -1)[None]
+    g = (g + rng.uniform(-0.6, 0.6, g.shape)).astype(np.float32)
+    for d in axes:
+        g[:, :, :, 16:, d] = value
+    x = rng.standard_normal((1, 4) + source).astype(np.float32)
+    u = rng.standard_normal((1, 4) + shape).astype(np.float32)
+    first = (Ellipsis, slice(0, 16))
+    g64, x64, u64 = (t.astype(np.float64) for t in (g[:, :, :, :16], x, u[first]))
+    for bound in ("zero", "dct2", "replicate"):
+        pull = G.grid_pull(T(x), T(g), [bound], [order], 1)
+        grad = G.grid_grad(T(x), T(g), [bound], [order], 1)
+        ggrad, = G.grid_pull_backward(T(u), T(x), T(g).requires_grad_(), [bound], [order], 1)
+        assert close(pull[first], O.grid_pull(x64, g64, bound, order, 1, oob_f32=True)), bound
+        assert close(grad[:, :, :, :, :16], O.grid_grad(x64, g64, bound, order, 1, oob_f32=True)), bound
+        ref = O.grid_pull_backward(u64, x64, g64, bound, order, 1, oob_f32=True)[1]
+        assert close(ggrad[:, :, :, :16], ref), bound
+        if bound == "zero" and np.isfinite(value):
+            assert not pull[..., 16:].any() and not grad[:, :, :, :, 16:].any() and not ggrad[:, :, :, 16:].any()
