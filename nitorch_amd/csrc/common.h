@@ -11,6 +11,7 @@
 #include <cstdint>
 #include <cmath>
 #include <mutex>
+#include <type_traits>
 
 #include "spline_tables.h"
 
@@ -73,56 +74,62 @@ enum BoundCode : int {
 // as zero").  In-range indices short-circuit (every bound maps them to
 // themselves with sign +1), so the integer modulo only runs on border taps.
 // The returned index is always in [0, n), also where the sign is 0, so that
-// an unguarded load through it stays inside the axis.
+// an unguarded load through it stays inside the axis -- for every value of
+// `i`: a coordinate beyond the integer range (or infinite) converts to its
+// limits, so the period's position is computed without a sum or a negation
+// that could overflow.
 // --------------------------------------------------------------------------
+// a mod m in [0, m)
+template <typename I, typename U = std::make_unsigned_t<I>>
+__host__ __device__ inline U pos_mod(I a, U m) {
+  const U r = (a < 0 ? ~U(a) : U(a)) % m;   // ~a = -a - 1
+  return a < 0 ? m - 1 - r : r;
+}
+
+// Tap t of a sample whose first tap is lo; wraps at the limits.
 template <typename I>
-__host__ __device__ inline I pos_mod(I a, I m) {
-  I r = a % m;
-  return r < 0 ? r + m : r;
+__host__ __device__ inline I tap_at(I lo, int t) {
+  using U = std::make_unsigned_t<I>;
+  return I(U(lo) + U(t));
 }
 
 template <typename I>
 __host__ __device__ inline I fold(int b, I i, I n, int &s) {
+  using U = std::make_unsigned_t<I>;
   s = 1;
   if (i >= 0 && i < n) return i;
+  const U m = U(n);
   switch (b) {
     case B_REPLICATE:
       return i < 0 ? I(0) : n - 1;
-    case B_DCT1: {
+    case B_DCT1: {   // mirrored about the end voxels
       if (n == 1) return 0;
-      I p = 2 * (n - 1);
-      I k = pos_mod<I>(i < 0 ? -i : i, p);
-      return k >= n ? p - k : k;
+      const U p = 2 * (m - 1), k = pos_mod<I>(i, p);
+      return I(k >= m ? p - k : k);
     }
-    case B_DCT2: {
-      I p = 2 * n;
-      I k = pos_mod<I>(i, p);
-      return k >= n ? p - 1 - k : k;
+    case B_DCT2: {   // mirrored about the ends
+      const U p = 2 * m, k = pos_mod<I>(i, p);
+      return I(k >= m ? p - 1 - k : k);
     }
     case B_DST2: {
-      I p = 2 * n;
-      I k = pos_mod<I>(i, p);
-      I j = i < 0 ? n - i - 1 : i;
-      s = ((j / n) & 1) ? -1 : 1;
-      return k >= n ? p - 1 - k : k;
+      const U p = 2 * m, k = pos_mod<I>(i, p);
+      if (k < m) return I(k);
+      s = -1;
+      return I(p - 1 - k);
     }
-    case B_DST1: {
+    case B_DST1: {   // mirrored about the voxels outside the ends, which read as zero
       if (n == 1) return 0;
-      I p = 2 * (n + 1);
-      I j = i < 0 ? n - i - 1 : i;
-      j = j % p;
-      if (j % (n + 1) == n) {   // between two reflections: reads as zero
+      const U p = 2 * (m + 1), k = pos_mod<I>(i, p);
+      if (k < m) return I(k);
+      if (k == m || k == p - 1) {
         s = 0;
         return 0;
       }
-      s = ((j / (n + 1)) & 1) ? -1 : 1;
-      I k = (i == -1) ? I(0) : (i < 0 ? -i - 2 : i);
-      k = pos_mod<I>(k, p);
-      if (k == n) return n - 1;
-      return k > n ? p - k - 2 : k;
+      s = -1;
+      return I(p - 2 - k);
     }
     case B_DFT:
-      return pos_mod<I>(i, n);
+      return I(pos_mod<I>(i, m));
     default:  // zero / nocheck / sliding: outside reads as zero
       s = 0;
       return 0;

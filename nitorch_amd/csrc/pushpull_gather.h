@@ -37,7 +37,7 @@ __device__ __forceinline__ unsigned ga_fold(int bound, int lo, int n, int stride
 #pragma unroll 1
   for (int t = 0; t <= ORD; ++t) {
     int s;
-    const int j = fold<int>(bound, lo + t, n, s) * stride;
+    const int j = fold<int>(bound, tap_at(lo, t), n, s) * stride;
     ok |= s != 0 ? 1u << t : 0u;
     tl_rot(of);
     tl_rot(w);

@@ -391,7 +391,7 @@ __global__ __launch_bounds__(256) void gtile_kernel(PPArgs<float> a, int ntx, in
         const int bd = k == 0 ? a.bound[0] : k == 1 ? a.bound[1] : a.bound[2];
         const int st = (int)(k == 0 ? a.src_s[2] : k == 1 ? a.src_s[3] : a.src_s[4]);
         int sg;
-        const int j = fold<int>(bd, m + b, nn, sg);
+        const int j = fold<int>(bd, tap_at(m, b), nn, sg);
         fofs[i] = j * st;
         fsg[i] = (float)sg;
       } else if (b == 0) {

@@ -195,7 +195,7 @@ __device__ __forceinline__ void pp_sample(const PPArgs<T> &a, I n, I w, I h, I d
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
         int s;
-        I j = fold<I>(a.bound[k], j0 + t, ssz[k], s);
+        I j = fold<I>(a.bound[k], tap_at(j0, t), ssz[k], s);
         ts[k][t] = s;
         ti[k][t] = j * src_sd[k];
         to[k][t] = j * out_sd[k];
@@ -205,7 +205,7 @@ __device__ __forceinline__ void pp_sample(const PPArgs<T> &a, I n, I w, I h, I d
 #pragma unroll
       for (int t = 0; t < MAXT; ++t) {
         if (ORD < 0 && t > ok) break;
-        const I b = lo + t;
+        const I b = tap_at(lo, t);
         const T dd = x - T(b);
         if (ok >= 1 && (t == 0 || t == ok)) {   // last piece, from x itself
           const T s = spl_outer_s<T, I>(ok, t, x, lo);

@@ -266,7 +266,7 @@ __global__ __launch_bounds__((STile<ORD>::NTH), 4) void scatter_kernel(PPArgs<fl
         const int b = q - (d == 0 ? 0 : (d == 1 ? e0 : e0 + e1));
         int sg = 0;
         const int j = fold<int>(d == 0 ? a.bound[0] : (d == 1 ? a.bound[1] : a.bound[2]),
-                                (d == 0 ? m0 : (d == 1 ? m1 : m2)) + b, d == 0 ? sz[0] : (d == 1 ? sz[1] : sz[2]), sg);
+                                tap_at(d == 0 ? m0 : (d == 1 ? m1 : m2), b), d == 0 ? sz[0] : (d == 1 ? sz[1] : sz[2]), sg);
         fofs[q] = j * (int)(d == 0 ? a.out_s[2] : (d == 1 ? a.out_s[3] : a.out_s[4]));
         fsg[q] = (float)sg;
       }

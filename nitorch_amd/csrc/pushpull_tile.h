@@ -411,7 +411,7 @@ __global__ __launch_bounds__((TileBox<ORD>::NTH),
       const int nn = d == 0 ? sz[0] : d == 1 ? sz[1] : sz[2];
       const int bd = d == 0 ? a.bound[0] : d == 1 ? a.bound[1] : a.bound[2];
       int sg = 0, j = 0;
-      if (b < e) j = fold<int>(bd, m + b, nn, sg);
+      if (b < e) j = fold<int>(bd, tap_at(m, b), nn, sg);
       fofs[i] = j * (d == 0 ? st0 : d == 1 ? st1 : st2);
       fsg[i] = (float)sg;
     }
@@ -745,7 +745,7 @@ __global__ __launch_bounds__(DYN_NTH) void tile_dyn(PPArgs<float> a, int ntx, in
         const int d = i < ext[0] ? 0 : (i < ext[0] + ext[1] ? 1 : 2);
         const int b = i - (d == 0 ? 0 : (d == 1 ? ext[0] : ext[0] + ext[1]));
         int sg = 0;
-        const int jj = fold<int>(a.bound[d], mn[d] + b, sz[d], sg);
+        const int jj = fold<int>(a.bound[d], tap_at(mn[d], b), sz[d], sg);
         fofs[i] = jj * (int)st[2 + d];
         fsg[i] = (float)sg;
       }

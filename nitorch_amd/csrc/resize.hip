@@ -65,7 +65,7 @@ __device__ inline int rs_taps(const RsArgs &a, int d, int w, long long stride, T
 #pragma unroll
   for (int t = 0; t < RS_MAXT; ++t) {
     if (t > o) break;
-    const int b = lo + t;
+    const int b = tap_at(lo, t);
     T g, h;
     spl_eval<T>(o, t, x - T(b), wt[t], g, h);
     int s;

@@ -140,7 +140,7 @@ __device__ __forceinline__ void svf_pull(const T *f, const SvfGeo &G, const int 
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       int s;
-      of[d][t] = fold<int>(G.bound[d], lo[d] + t, G.n[d], s) * st[d];
+      of[d][t] = fold<int>(G.bound[d], tap_at(lo[d], t), G.n[d], s) * st[d];
       on[d][t] = s != 0;
       ws[d][t] = s < 0 ? -w[d][t] : w[d][t];
     }
@@ -226,9 +226,9 @@ __global__ __launch_bounds__(SV3_BLOCK) void svf_step(SvfGeo G, int64_t nvox, co
     int s;
 #pragma unroll
     for (int a = 0; a < 4; ++a) {
-      ix[a] = (inner ? lo[0] - 1 + a : fold<int>(B_DFT, lo[0] - 1 + a, G.n[0], s)) * sx;
-      iy[a] = (inner ? lo[1] - 1 + a : fold<int>(B_DFT, lo[1] - 1 + a, G.n[1], s)) * sy;
-      iz[a] = (inner ? lo[2] - 1 + a : fold<int>(B_DFT, lo[2] - 1 + a, G.n[2], s)) * 3;
+      ix[a] = (inner ? lo[0] - 1 + a : fold<int>(B_DFT, tap_at(lo[0], a - 1), G.n[0], s)) * sx;
+      iy[a] = (inner ? lo[1] - 1 + a : fold<int>(B_DFT, tap_at(lo[1], a - 1), G.n[1], s)) * sy;
+      iz[a] = (inner ? lo[2] - 1 + a : fold<int>(B_DFT, tap_at(lo[2], a - 1), G.n[2], s)) * 3;
     }
     T J[3][3];   // [component][axis], pulled central differences
 #pragma unroll

@@ -47,3 +47,48 @@ def test_axis_inside(helpers):
     out = helpers("axis_inside((int)a[0], (int)a[1], (int)a[2])", args)
     first, extent, n = args.T
     assert np.array_equal(out.astype(bool), (first >= 0) & (first + extent <= n))
+
+
+def fold_reference(bound, i, n):
+    """Index and sign of voxel i under a bound's periodic extension, from the
+    definition, in exact integers."""
+    if 0 <= i < n:
+        return i, 1
+    if bound == 0:
+        return min(max(i, 0), n - 1), 1
+    if bound == 1:
+        k = i % (2 * n - 2) if n > 1 else 0
+        return (k, 1) if k < n else (2 * n - 2 - k, 1)
+    if bound in (2, 4):
+        k = i % (2 * n)
+        return (k, 1) if k < n else (2 * n - 1 - k, 1 if bound == 2 else -1)
+    if bound == 3:
+        if n == 1:
+            return 0, 1
+        k = i % (2 * n + 2)
+        if k in (n, 2 * n + 1):
+            return 0, 0
+        return (k, 1) if k < n else (2 * n - k, -1)
+    return (i % n, 1) if bound == 5 else (0, 0)
+
+
+@pytest.mark.parametrize("width", [32, 64])
+def test_fold(helpers, width):
+    lo, hi = -2 ** (width - 1), 2 ** (width - 1) - 1
+    ends = list(range(70)) + [97, 100, 1000, 65535, 10 ** 6]
+    at = sorted(set([lo + e for e in ends] + [hi - e for e in ends] + list(range(-200, 201))))
+    args = np.array([(b, i, n) for b in range(9) for n in list(range(1, 13)) + [16, 30, 32, 62, 97, 181, 2 ** 30 + 1]
+                     for i in at])
+    kind = "int" if width == 32 else "int64_t"
+    out = helpers(f"({{ int s; long long j = fold<{kind}>((int)a[0], ({kind})a[1], ({kind})a[2], s);"
+                  " j * 4 + s + 1; })", args)
+    ref = [4 * j + s + 1 for j, s in (fold_reference(*(int(v) for v in row)) for row in args)]
+    assert np.array_equal(out, np.array(ref))
+    n = args[:, 2]
+    assert ((out >> 2 >= 0) & (out >> 2 < n)).all()
+
+
+def test_tap_at(helpers):
+    args = np.array([(f, t) for f in (IMIN, -1, 0, 7, IMAX - 7, IMAX) for t in range(8)])
+    out = helpers("tap_at((int)a[0], (int)a[1])", args)
+    assert np.array_equal(out, (args.sum(1) + 2 ** 31) % 2 ** 32 - 2 ** 31)

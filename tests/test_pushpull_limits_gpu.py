@@ -40,7 +40,7 @@ def test_gather_beyond_the_integer_range(order, axes, value):
     u = rng.standard_normal((1, 4) + shape).astype(np.float32)
     first = (Ellipsis, slice(0, 16))
     g64, x64, u64 = (t.astype(np.float64) for t in (g[:, :, :, :16], x, u[first]))
-    for bound in ("zero", "dct2", "replicate"):
+    for bound in ("zero", "dct1", "dct2", "dst1", "dst2", "dft", "replicate"):
         pull = G.grid_pull(T(x), T(g), [bound], [order], 1)
         grad = G.grid_grad(T(x), T(g), [bound], [order], 1)
         ggrad, = G.grid_pull_backward(T(u), T(x), T(g).requires_grad_(), [bound], [order], 1)
