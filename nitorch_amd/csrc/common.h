@@ -136,6 +136,13 @@ __host__ __device__ inline I fold(int b, I i, I n, int &s) {
   }
 }
 
+// Place of i among the n positions -off, -off + 1, ..., or -1 when it is none
+// of them (for every integer i).
+__host__ __device__ inline int place_in(int i, int off, int n) {
+  const unsigned p = unsigned(i) + unsigned(off);
+  return p < unsigned(n) ? int(p) : -1;
+}
+
 // Whether positions first .. first + extent - 1 all lie in [0, n).  (`first`
 // may be any integer: `first + extent` could overflow.)
 __host__ __device__ inline bool axis_inside(int first, int extent, int n) { return first >= 0 && first <= n - extent; }

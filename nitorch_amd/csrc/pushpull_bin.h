@@ -84,8 +84,9 @@ __device__ __forceinline__ bool bin_taps(const PPArgs<float> &a, int n, int px, 
 
 // Bin of first taps lo, or -1 when lo is outside the binned range.
 __device__ __forceinline__ int64_t bin_of(const int (&lo)[3], int n, int nbx, int nby, int nbz) {
-  const int bx = lo[0] + BIN_OFF, by = lo[1] + BIN_OFF, bz = lo[2] + BIN_OFF;
-  if (bx < 0 || by < 0 || bz < 0 || bx >= nbx * BIN_S || by >= nby * BIN_S || bz >= nbz * BIN_S) return -1;
+  const int bx = place_in(lo[0], BIN_OFF, nbx * BIN_S), by = place_in(lo[1], BIN_OFF, nby * BIN_S),
+            bz = place_in(lo[2], BIN_OFF, nbz * BIN_S);
+  if (bx < 0 || by < 0 || bz < 0) return -1;
   return (((int64_t)n * nbx + bx / BIN_S) * nby + by / BIN_S) * nbz + bz / BIN_S;
 }
 

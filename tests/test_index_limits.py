@@ -92,3 +92,12 @@ def test_tap_at(helpers):
     args = np.array([(f, t) for f in (IMIN, -1, 0, 7, IMAX - 7, IMAX) for t in range(8)])
     out = helpers("tap_at((int)a[0], (int)a[1])", args)
     assert np.array_equal(out, (args.sum(1) + 2 ** 31) % 2 ** 32 - 2 ** 31)
+
+
+def test_place_in(helpers):
+    """The range test of the first-tap bins."""
+    at = [IMIN, IMIN + 1, IMIN + 8, -9, -8, -1, 0, 1, 7, 23, 24, 183, 184, IMAX - 8, IMAX - 7, IMAX - 1, IMAX]
+    args = np.array([(i, 8, n) for i in at for n in (8, 32, 192, 2 ** 20)])
+    out = helpers("place_in((int)a[0], (int)a[1], (int)a[2])", args)
+    place = args[:, 0] + args[:, 1]
+    assert np.array_equal(out, np.where((place >= 0) & (place < args[:, 2]), place, -1))
