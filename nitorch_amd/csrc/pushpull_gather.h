@@ -28,7 +28,8 @@ namespace ni_amd {
 
 // Folded offsets and signed weights of one axis's taps.  Bit t of `ok` is
 // set when tap t lies inside (sign != 0): a tap that reads as zero must not
-// let its voxel's value through (it may be a NaN).
+// let its voxel's value through (it may be a NaN), nor its weight (infinite
+// or NaN at an infinite coordinate).
 template <int ORD, bool DERIV>
 __device__ __forceinline__ unsigned ga_fold(int bound, int lo, int n, int stride, float (&w)[ORD + 1],
                                             float (&g)[ORD + 1], int (&of)[ORD + 1]) {
@@ -42,10 +43,10 @@ __device__ __forceinline__ unsigned ga_fold(int bound, int lo, int n, int stride
     tl_rot(of);
     tl_rot(w);
     of[ORD] = j;
-    w[ORD] *= (float)s;
+    w[ORD] = s != 0 ? w[ORD] * (float)s : 0.f;
     if constexpr (DERIV) {
       tl_rot(g);
-      g[ORD] *= (float)s;
+      g[ORD] = s != 0 ? g[ORD] * (float)s : 0.f;
     }
   }
   return ok;

@@ -22,6 +22,8 @@
 
 namespace ni_amd {
 
+#define FAR_TAP (1 << 30)   // first taps beyond are a saturated conversion's
+
 // ONE: single-channel calls, whose kernels need fewer registers.
 template <int ORD, bool DERIV, bool ONE>
 struct GTile {
@@ -354,7 +356,9 @@ __global__ __launch_bounds__(256) void gtile_kernel(PPArgs<float> a, int ntx, in
     mx[k] = __builtin_amdgcn_readfirstlane(mx[k]);
     none = none || mn[k] > mx[k];
     const int64_t e = (int64_t)mx[k] - (int64_t)mn[k] + NT;
-    fits = fits && e <= B::MAXE;
+    // (coordinates beyond the integer range have weights that a staged zero
+    // would not cancel: ga_sample drops them)
+    fits = fits && e <= B::MAXE && mn[k] > -FAR_TAP && mx[k] < FAR_TAP;
     d.e[k] = (int)(e <= B::MAXE ? e : B::MAXE);
   }
   // no in-bound sample: one channel of an (unread) unit box, so that the

@@ -79,3 +79,36 @@ def test_bins_beyond_the_integer_range(order):
     count = G.grid_count(T(g), list(shape), ["zero"], [order], 1).cpu().double().numpy()
     ref = O.grid_count(g64, shape, "zero", order, 1, oob_f32=True)
     assert (np.abs(count - ref) <= 1e-4 * ref + 1e-36).all()
+
+
+@pytest.mark.parametrize("order", [0, 1, 2, 3, 5, 7])
+@pytest.mark.parametrize("channels", [1, 4])
+def test_infinite_coordinates_read_as_zero(order, channels):
+    """Under `zero`, samples beyond the integer range or infinite along an
+    axis read as zero whatever their weights (infinite or NaN there), alone
+    in their tile and as whole tiles."""
+    from nitorch_amd import grid as G
+    rng = np.random.default_rng(10 * order + channels)
+    shape, source = (8, 8, 48), (9, 10, 50)
+    g = np.stack(np.meshgrid(*[np.arange(n, dtype=np.float64) for n in shape], indexing="ij"), -1)[None]
+    g = (g + rng.uniform(-0.6, 0.6, g.shape)).astype(np.float32)
+    values = [3e9, 1e10, -1e10, 1e30, np.inf, -np.inf]
+    g[0, 1, 2, 16:32] = np.inf
+    g[0, 1:3, 3, 5, 1] = -np.inf
+    g[0, 4, 4, 16:20, 2] = 1e10
+    for k, v in enumerate(values):   # whole tiles of 4 x 8 x 16
+        h = g.copy()
+        h[0, :4, :, 32:, k % 3] = v
+        h[0, 4:, :, :16] = v
+        h64 = np.nan_to_num(h.astype(np.float64), posinf=1e10, neginf=-1e10).clip(-1e10, 1e10)
+        x = rng.standard_normal((1, channels) + source).astype(np.float32)
+        u = rng.standard_normal((1, channels) + shape).astype(np.float32)
+        x64, u64 = x.astype(np.float64), u.astype(np.float64)
+        pull = G.grid_pull(T(x), T(h), ["zero"], [order], 1)
+        assert close(pull, O.grid_pull(x64, h64, "zero", order, 1, oob_f32=True)), v
+        if order == 0:
+            continue
+        grad = G.grid_grad(T(x), T(h), ["zero"], [order], 1)
+        assert close(grad, O.grid_grad(x64, h64, "zero", order, 1, oob_f32=True)), v
+        ggrad, = G.grid_pull_backward(T(u), T(x), T(h).requires_grad_(), ["zero"], [order], 1)
+        assert close(ggrad, O.grid_pull_backward(u64, x64, h64, "zero", order, 1, oob_f32=True)[1]), v
