@@ -379,8 +379,9 @@ __global__ __launch_bounds__(256) void gtile_kernel(PPArgs<float> a, int ntx, in
     return;
   }
   d.DYZ = gt_plane<B::CAP>(d.e[0], d.e[1], d.e[2], ncc);
-  // (32-bit byte offsets of a plane position: 2 * 64 strides below 2^31)
-  d.inner = !none && a.src_s[3] < (1 << 22) && a.src_s[4] < (1 << 22);
+  // (unsigned 32-bit byte offsets of a plane position: 2 * 64 strides below
+  // 2^31, and none that steps back, as a flipped view's do)
+  d.inner = !none && (uint64_t)a.src_s[3] < (1u << 22) && (uint64_t)a.src_s[4] < (1u << 22);
 #pragma unroll
   for (int k = 0; k < 3; ++k) d.inner = d.inner && axis_inside(mn[k], d.e[k], sz[k]);
   d.base = mn[0] * (int)a.src_s[2] + mn[1] * (int)a.src_s[3] + mn[2] * (int)a.src_s[4];

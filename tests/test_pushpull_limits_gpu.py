@@ -1,9 +1,11 @@
 """GPU checks of pulls at the limits of what their entry points take:
 extrapolated coordinates beyond the integer range or infinite, whose first
-taps saturate.
+taps saturate, and source views with negative strides (C ABI).
 
 Tolerance against the FP64 oracle: 1e-5 norm-relative, as the other gathers
 (float sums of at most (order + 1)^3 terms)."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -112,3 +114,30 @@ def test_infinite_coordinates_read_as_zero(order, channels):
         assert close(grad, O.grid_grad(x64, h64, "zero", order, 1, oob_f32=True)), v
         ggrad, = G.grid_pull_backward(T(u), T(x), T(h).requires_grad_(), ["zero"], [order], 1)
         assert close(ggrad, O.grid_pull_backward(u64, x64, h64, "zero", order, 1, oob_f32=True)[1]), v
+
+
+@pytest.mark.parametrize("order", [0, 1, 2, 3, 5])
+@pytest.mark.parametrize("channels", [1, 4])
+@pytest.mark.parametrize("flip", [(4,), (3,), (2,), (3, 4), (1, 2, 3, 4)])
+def test_flipped_source_views(order, channels, flip):
+    """A source whose strides are negative along some dims reads as its
+    flipped copy, bit for bit; most tiles of 4 x 8 x 16 lie well inside it."""
+    from nitorch_amd import _lib as L
+    from nitorch_amd import grid as G
+    rng = np.random.default_rng(order)
+    shape, source = (8, 16, 32), (20, 28, 44)
+    g = np.stack(np.meshgrid(*[np.arange(n, dtype=np.float64) for n in shape], indexing="ij"), -1)[None]
+    g = T((g + 6 + rng.uniform(-0.6, 0.6, g.shape)).astype(np.float32))
+    x = T(rng.standard_normal((1, channels) + source).astype(np.float32))
+    strides = list(x.stride())
+    first = sum((x.shape[d] - 1) * strides[d] for d in flip)
+    view = [-s if d in flip else s for d, s in enumerate(strides)]
+    b, o = L.i32arr([2] * 3), L.i32arr([order] * 3)
+    for name, ref in (("grid_pull", G.grid_pull), ("grid_grad", G.grid_grad)):
+        ref = ref(x.flip(flip), g, ["dct2"], [order], 0)
+        out = torch.full_like(ref, 7.0)
+        L.check(getattr(L.lib(), "ni_" + name)(
+            L.dtype_code(x.dtype), 3, b, o, 0, 1, channels, L.i64arr(source), L.i64arr(shape),
+            ctypes.c_void_p(x.data_ptr() + 4 * first), L.i64arr(view), L.ptr(g), L.strides(g), L.ptr(out),
+            L.strides(out), L.stream_of(g)), name)
+        assert torch.equal(out, ref), name
