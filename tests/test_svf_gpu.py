@@ -211,3 +211,26 @@ def test_fused_squarings_leave_transforms_and_strides_alone():
     assert rel(svf.exp_forward(chan_first, steps=3), svf.exp_forward(v, steps=3).cpu().numpy()) <= 1e-12
     with FA.dual_level(), pytest.raises((RuntimeError, NotImplementedError)):
         svf.exp_forward(FA.make_dual(v, torch.ones_like(v)), steps=2)
+
+
+@pytest.mark.parametrize("offset", [0.0, 60.0])
+def test_fused_squaring_of_a_translation_part(offset):
+    """A constant part of tens of voxels does not reach the Jacobian's
+    rounding.  One squaring of u (at most 30.2 voxels), FP32 against FP64 on
+    the same values: the sampled position carries half an ulp of 64, 1.9e-6,
+    times the Jacobian's slope (u'' <= 0.03 an axis, 3 axes: 1.7e-7), and an
+    entry of about 1 a few roundings of 6e-8: 1e-6.  (Differences of the
+    velocities themselves carry roundings of 30: 3e-6.)"""
+    from nitorch_amd import svf
+    shape = (24, 20, 28)
+    v = (_vel(shape, 0.2, 31) + offset * np.array([1.0, -0.9, 0.8])).astype(np.float32)
+    _, ref = E.exp_forward_jac(v.astype(np.float64), steps=1)
+    _, jac = svf.exp_forward(torch.from_numpy(v).to(DEV), steps=1, displacement=True, jacobian=True)
+    assert np.abs(jac.cpu().double().numpy() - ref).max() <= 1e-6
+    g = _vel(shape, 1.0, 32)
+    gref = E.exp_backward(v.astype(np.float64), g.astype(np.float32).astype(np.float64), steps=1, rotate_grad=True)
+    out = svf.exp_backward(torch.from_numpy(v).to(DEV), torch.from_numpy(g).float().to(DEV), steps=1,
+                           rotate_grad=True)
+    # the gradient is pulled at that position too (slope <= 0.5 an axis: 3e-6)
+    # and passes through two Jacobians
+    assert rel(out, gref) <= 1e-5
