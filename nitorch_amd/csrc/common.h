@@ -136,6 +136,11 @@ __host__ __device__ inline I fold(int b, I i, I n, int &s) {
   }
 }
 
+// Whether fold can return a sign other than +1.
+__host__ __device__ inline bool bound_signs(int b) {
+  return !(b == B_REPLICATE || b == B_DCT1 || b == B_DCT2 || b == B_DFT);
+}
+
 // Place of i among the n positions -off, -off + 1, ..., or -1 when it is none
 // of them (for every integer i).
 __host__ __device__ inline int place_in(int i, int off, int n) {

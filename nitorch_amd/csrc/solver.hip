@@ -660,9 +660,9 @@ __global__ __launch_bounds__(relax_small_threads<T>()) void relax_small(T *__res
   }
   __syncthreads();
   const int *ftx = ft, *fty = ft + 5 * G.X, *ftz = ft + 5 * (G.X + G.Y);
-  // folds that flip signs or zero values: dst1, dst2, zero
+  // folds that flip signs or zero values
   bool signs = false;
-  for (int d = 0; d < 3; ++d) signs = signs || G.b[d] == B_DST1 || G.b[d] == B_DST2 || G.b[d] == B_ZERO;
+  for (int d = 0; d < 3; ++d) signs = signs || bound_signs(G.b[d]);
   for (int it = 0; it < nb_iter; ++it)
     for (int col = 0; col < ncls; ++col) {
       const int c0 = start[col], cn = start[col + 1] - c0;

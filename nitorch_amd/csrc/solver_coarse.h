@@ -262,7 +262,7 @@ struct Coarse {
 
   __device__ __forceinline__ Coarse(const CoarseArgs<T> &a_, CoarseLds<T, CG> &m_) : a(a_), m(m_), n((int)blockIdx.x), flip(0) {
     signs = false;
-    for (int d = 0; d < 3; ++d) signs = signs || a.b[d] == B_DST1 || a.b[d] == B_DST2 || a.b[d] == B_ZERO;
+    for (int d = 0; d < 3; ++d) signs = signs || bound_signs(a.b[d]);
   }
   __device__ __forceinline__ int vox(const CoarseLevel<T> &L) const { return L.X * L.Y * L.Z; }
 

@@ -101,3 +101,10 @@ def test_place_in(helpers):
     out = helpers("place_in((int)a[0], (int)a[1], (int)a[2])", args)
     place = args[:, 0] + args[:, 1]
     assert np.array_equal(out, np.where((place >= 0) & (place < args[:, 2]), place, -1))
+
+
+def test_bound_signs(helpers):
+    args = np.array([(b, i, 5) for b in range(9) for i in range(-40, 41)])
+    sign = helpers("({ int s; fold<int>((int)a[0], (int)a[1], (int)a[2], s); (long long)s; })", args).reshape(9, -1)
+    named = helpers("bound_signs((int)a[0])", np.arange(9)[:, None])
+    assert np.array_equal(named.astype(bool), (sign != 1).any(1))

@@ -316,3 +316,18 @@ def test_fmg_coarse_levels_vs_oracle(sv, case, use_cg):
     ref = S.fmg_grid(h, g, bound=bound, nb_cycles=2, nb_iter=2, **kw, **p)
     tol = (2e-4 if use_cg else 1e-4) if dt == torch.float32 else 1e-9
     assert rel(x, ref) <= tol, case
+
+
+@pytest.mark.parametrize("use_cg", [False, True])
+@pytest.mark.parametrize("code", [6, 8])
+@pytest.mark.parametrize("shape", [(11, 9, 10), (21, 18, 22)])
+def test_fmg_unnamed_zero_bounds(sv, monkeypatch, shape, code, use_cg):
+    """The bound codes without a name (sliding, nocheck) fold as `zero` on
+    every level of a pyramid."""
+    from nitorch_amd import _lib as L
+    rng = np.random.default_rng(62)
+    g, h = system(rng, shape, CC=6, N=1)
+    args = (T(h, torch.float64), T(g, torch.float64), None, pen_vec(PENS[3]), (1, 1, 1), "zero", 2, 2)
+    ref = sv.fmg_grid_cf(*args, use_cg=use_cg).cpu().numpy()
+    monkeypatch.setattr(sv, "_bounds", lambda bound: L.i32arr([code] * 3))
+    assert rel(sv.fmg_grid_cf(*args, use_cg=use_cg), ref) <= 1e-9
