@@ -287,6 +287,10 @@ __host__ __device__ inline void spl_outer_rt(int order, bool left, T s, T &w, T 
   }
 }
 
+// A launch counts its work-items along x in 32 bits: a larger grid wraps, and
+// runs in part without an error.
+inline bool launch_fits(int64_t blocks, int64_t threads) { return blocks * threads < int64_t(1) << 32; }
+
 // --------------------------------------------------------------------------
 // Error reporting for the C ABI.
 // --------------------------------------------------------------------------

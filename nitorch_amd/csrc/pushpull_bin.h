@@ -532,7 +532,7 @@ static inline bool bin_plan(const PPArgs<float> &a, int64_t ntiles, int TS, BinP
   p.nbz = (int)((a.sZ + 2 * BIN_OFF + BIN_S - 1) / BIN_S);
   p.nbins = a.N * (int64_t)p.nbx * p.nby * p.nbz;
   p.nsamp = ntiles * TS;   // listed samples, at most
-  if (p.nbins >= (int64_t(1) << 31) || p.nsamp >= (int64_t(1) << 31)) return false;
+  if (!launch_fits(p.nbins, BIN_NTH) || p.nsamp >= (int64_t(1) << 31)) return false;
   int *mem = nullptr;
   if (scratch_alloc((void **)&mem, sizeof(int) * (size_t)(2 * p.nbins + 5 + 2 * ntiles + p.nsamp), st) != hipSuccess) {
     (void)hipGetLastError();

@@ -438,26 +438,20 @@ template <int ORD> constexpr bool direct_scatter() { return ORD == 0; }
 #define NI_DEFINE_DISPATCH_ORDER(ORD)                                            \
   template <> bool dispatch_order<ORD>(const PPArgs<float> &a, int64_t total, hipStream_t st) { \
     switch (a.flags) {                                                          \
-      case F_PULL: launch_tile<ORD, TM_PULL>(a, st); return true;               \
-      case F_SGRAD: launch_tile<ORD, TM_SGRAD>(a, st); return true;             \
+      case F_PULL: return launch_tiles<ORD, TM_PULL>(a, st);                    \
+      case F_SGRAD: return launch_tiles<ORD, TM_SGRAD>(a, st);                  \
       case F_PUSH | F_TRGT:                                                     \
-        if constexpr (direct_scatter<ORD>())                                    \
-          launch_fast<float, int32_t, ORD, F_PUSH | F_TRGT>(a, total, st);      \
-        else                                                                    \
-          launch_tile<ORD, TM_PUSH>(a, st);                                     \
+        if constexpr (!direct_scatter<ORD>()) return launch_tiles<ORD, TM_PUSH>(a, st); \
+        launch_fast<float, int32_t, ORD, F_PUSH | F_TRGT>(a, total, st);        \
         return true;                                                            \
       case F_COUNT:                                                             \
-        if constexpr (direct_scatter<ORD>())                                    \
-          launch_fast<float, int32_t, ORD, F_COUNT>(a, total, st);              \
-        else                                                                    \
-          launch_tile<ORD, TM_COUNT>(a, st);                                    \
+        if constexpr (!direct_scatter<ORD>()) return launch_tiles<ORD, TM_COUNT>(a, st); \
+        launch_fast<float, int32_t, ORD, F_COUNT>(a, total, st);                \
         return true;                                                            \
-      case F_PUSH | F_GRAD | F_TRGT:                                            \
-        launch_tile<ORD, TM_PUSH>(a, st); launch_tile<ORD, TM_GGRAD>(a, st); return true; \
-      case F_GRAD | F_TRGT: launch_tile<ORD, TM_GGRAD>(a, st); return true;     \
-      case F_PULL | F_GRAD | F_TRGT:                                            \
-        launch_tile<ORD, TM_PULL>(a, st); launch_tile<ORD, TM_GGRAD>(a, st); return true; \
-      case F_GRAD: launch_tile<ORD, TM_GGRAD1>(a, st); return true;             \
+      case F_PUSH | F_GRAD | F_TRGT: return launch_tiles<ORD, TM_PUSH, TM_GGRAD>(a, st); \
+      case F_GRAD | F_TRGT: return launch_tiles<ORD, TM_GGRAD>(a, st);          \
+      case F_PULL | F_GRAD | F_TRGT: return launch_tiles<ORD, TM_PULL, TM_GGRAD>(a, st); \
+      case F_GRAD: return launch_tiles<ORD, TM_GGRAD1>(a, st);                  \
       default: return false;                                                    \
     }                                                                           \
   }

@@ -837,6 +837,17 @@ static void launch_gather_mode(const PPArgs<float> &a, hipStream_t st) {
   if constexpr (ORD > 0) launch_gtile<ORD, MODE>(a, nullptr, st);
 }
 
+// Whether the mode's first kernel can cover the samples in one launch (thin or
+// very many lattices leave most of a block idle, up to 255 of 256 threads).
+template <int ORD, int MODE>
+static bool tile_fits(const PPArgs<float> &a) {
+  using B = TileDims<ORD, MODE>;
+  const bool cache = TileMeta<MODE>::gather && a.C <= gather_channels<ORD, MODE>();
+  const int64_t bx = cache ? GA_TX : B::TX, by = cache ? GA_TY : B::TY, bz = cache ? GA_TZ : B::TZ;
+  return launch_fits(a.N * ((a.tX + bx - 1) / bx) * ((a.tY + by - 1) / by) * ((a.tZ + bz - 1) / bz),
+                     TileMeta<MODE>::gather ? GA_NTH : TileBox<ORD>::NTH);
+}
+
 // Push / count: tile_kernel, then the tiles it listed as too scattered.  In
 // calls of at least BIN_MIN_SAMPLES samples that may allocate: scatter_kernel
 // on those that fit a few larger boxes, the binned pass on the others.
@@ -883,6 +894,14 @@ static void launch_tile(const PPArgs<float> &a, hipStream_t st) {
       hipLaunchKernelGGL((tile_fallback<ORD, MODE>), g, b, 0, st, a, ntx, nty, ntz, nb, (const int *)nullptr);
     }
   }
+}
+
+// Every mode of a call, or false (nothing launched) if one does not fit.
+template <int ORD, int... MODES>
+static bool launch_tiles(const PPArgs<float> &a, hipStream_t st) {
+  if (!(tile_fits<ORD, MODES>(a) && ...)) return false;
+  (launch_tile<ORD, MODES>(a, st), ...);
+  return true;
 }
 
 }  // namespace ni_amd

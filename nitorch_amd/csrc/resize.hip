@@ -620,7 +620,7 @@ static bool rs_fused(const T *input, T *output, const RsArgs &a, hipStream_t st)
   const int txo = tall ? 16 : 4;
   const int ntx = (a.nt[0] + txo - 1) / txo;
   const long long nb = per * ntx;
-  if (nb >= (1LL << 31)) return false;
+  if (!launch_fits(nb, RS_BLOCK)) return false;
   const dim3 g((unsigned)nb), b(RS_BLOCK);
 #define RF_LAUNCH(TX, M) \
   hipLaunchKernelGGL((resize_fused<T, TX, M>), g, b, 0, st, input, output, a, ntx, nty, ntz, (unsigned)nb)
@@ -731,7 +731,7 @@ int ni_affine_grid(int32_t dtype, int64_t nbatch, const int64_t *shape, const vo
   }
   const long long n = nbatch * V;
   if (n <= 0) return 0;
-  NI_CHECK((n + RS_BLOCK - 1) / RS_BLOCK < (1LL << 31) - 1, "affine_grid: lattice too large");
+  NI_CHECK(launch_fits((n + RS_BLOCK - 1) / RS_BLOCK, RS_BLOCK), "affine_grid: lattice too large");
   hipStream_t st = (hipStream_t)stream;
   if (dtype == NI_FLOAT32)
     hipLaunchKernelGGL(affine_lattice<float>, dim3(rs_blocks(n)), dim3(RS_BLOCK), 0, st, (const float *)mat,

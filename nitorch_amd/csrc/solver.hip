@@ -1951,7 +1951,7 @@ static int fmg_setup(FMG<T> &F, int N, const int *sz, const T *hess, int CC, con
   // the coarse levels that one launch handles
   F.lc = F.NL;
   size_t co_vox = 0;
-  if (!has_w && coarse_ready<T>())
+  if (!has_w && launch_fits(N, CoarseCfg<T>::NTH) && coarse_ready<T>())
     while (F.lc > 0 && F.NL - F.lc < CO_LEVELS && F.L[F.lc - 1].V <= (size_t)CoarseCfg<T>::LIM &&
            F.L[F.lc - 1].sz[0] + F.L[F.lc - 1].sz[1] + F.L[F.lc - 1].sz[2] <= CO_AXES &&
            co_vox + F.L[F.lc - 1].V <= (size_t)CoarseCfg<T>::TAB &&

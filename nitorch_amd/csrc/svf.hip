@@ -389,7 +389,7 @@ static int svf_geo(int32_t dtype, int64_t N, const int64_t *shape, const int32_t
   G.nty = (G.n[1] + SVF_TY - 1) / SVF_TY;
   G.ntz = (G.n[2] + SVF_TZ - 1) / SVF_TZ;
   nb = N * (int64_t)G.ntx * G.nty * G.ntz;
-  NI_CHECK(nb < (int64_t(1) << 31) - 1, "svf: too many voxels");
+  NI_CHECK(launch_fits(nb, SV3_BLOCK), "svf: too many voxels");
   return 0;
 }
 

@@ -280,7 +280,8 @@ def _reslice_lattice(affine, affine_to, shape):
     else:
         a, b = affine.cpu(), affine_to.cpu()
     mat = affine_lmdiv(a, b)[..., :3, :]
-    if mat.shape[-2:] != (3, 4):
+    # (a launch counts its voxels in 32 bits)
+    if mat.shape[-2:] != (3, 4) or mat.shape[:-2].numel() * n >= 2 ** 32 - 256:
         return affine_grid(affine_lmdiv(affine, affine_to), shape)
     return _AffineLattice.apply(mat.contiguous().to(affine.device), shape)
 

@@ -226,12 +226,15 @@ def _fused(vel, interpolation, bound, *others):
     """Bound codes if the fused squarings apply to the velocity (and the
     contiguous fields `others` of its shape), else None: linear
     interpolation, 3-D contiguous float32 / float64 GPU fields, at least two
-    voxels along each axis (one has no difference to take) and 32-bit offsets
-    within a volume."""
+    voxels along each axis (one has no difference to take), 32-bit offsets
+    within a volume and 32-bit counts of work-items (blocks of 4 x 2 x 32
+    voxels, 256 each: thin lattices fill them in part)."""
     if not (vel.is_cuda and vel.dim() >= 4 and vel.shape[-1] == 3 and vel.dtype in (torch.float32, torch.float64)):
         return None
     shape = vel.shape[-4:-1]
     if min(shape) < 2 or 3 * shape[0] * shape[1] * shape[2] >= 2 ** 31 - 1 or vel.numel() == 0:
+        return None
+    if vel.shape[:-4].numel() * -(-shape[0] // 4) * -(-shape[1] // 2) * -(-shape[2] // 32) >= 2 ** 24:
         return None
     if any(int(o) != 1 for o in inter_to_nitorch(make_list(interpolation), "int")):
         return None
