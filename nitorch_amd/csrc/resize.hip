@@ -601,10 +601,54 @@ __global__ __launch_bounds__(RS_BLOCK) void resize_fused(const T *__restrict__ i
     if (ox0 + j < a.nt[0]) dst[j * oplane] = a.accumulate ? dst[j * oplane] + acc[j] : acc[j];
 }
 
+// Estimated time of a pass an axis, in us: elements written and taps, by the
+// kernel that the length and alignment of the rows select (16-byte rows, rows,
+// the contiguous axis, short rows), and never less than its six launches.
+template <typename T>
+static double rs_passes_time(const RsArgs &a, bool aligned) {
+  static const double f32[4][2] = {{1.8, 0.19}, {2.4, 0.61}, {1.6, 1.1}, {0, 0.37}};
+  static const double f64[4][2] = {{2.2, 0.44}, {2.8, 0.66}, {3.1, 1.5}, {0, 0.19}};
+  const bool f = sizeof(T) == 4;
+  double us = f ? 35 : 30, n = 1e-6 * a.N * a.C * (double)a.ns[0] * a.ns[1] * a.ns[2];
+  for (int d = 0; d < 3; ++d) {
+    long long B = 1;
+    for (int e = d + 1; e < 3; ++e) B *= a.ns[e];
+    n = n / a.ns[d] * a.nt[d];
+    const int kind = B >= 64 ? (B % 4 == 0 && aligned ? 0 : 1) : B == 1 ? 2 : 3;
+    const double(&c)[2] = (f ? f32 : f64)[kind];
+    us += n * (c[0] + c[1] * (a.order[d] + 1));
+  }
+  return std::max(us, 57.);
+}
+
+// Estimated time of resize_fused: per work-group, per plane that it walks, and
+// per plane for the rows summed along z, the values staged and the outputs
+// accumulated.
+template <typename T>
+static double rf_time(const RsArgs &a, bool wide, int txo, long long nb) {
+  // us per million: work-groups, planes, z rows / 8, values / 256, outputs, tap weights; us a launch
+  static const double cost[2][2][7] = {{{0, 270, 180, 16, 5, 12, 15}, {4000, 220, 200, 52, 23, 21, 25}},
+                                       {{520, 750, 230, 21, 0, 18, 8}, {4300, 0, 150, 45, 140, 68, 27}}};
+  const double(&c)[7] = cost[sizeof(T) == 8][wide];
+  const double b = 1e-6 * nb, np = rf_extent(a, 0, txo), ny = rf_extent(a, 1, RF_OY), nz = rf_extent(a, 2, RF_OZ);
+  return b * (c[0] + c[5] * txo * txo + np * (c[1] + c[2] * std::ceil(ny / RF_OY) + c[3] * ny * nz / RS_BLOCK +
+                                              c[4] * txo)) + c[6];
+}
+
 // One launch when the taps of a tile fit what the kernel stages: 3-D volumes
 // resized by a factor of about a third or more (2048 staged values: 8 x 32
 // outputs of a cubic half-size resize use 19 x 67), axes up to 2048, a sane
-// affine map.  False otherwise (the caller then runs a pass an axis).
+// affine map -- and the tiles are not mostly idle: a block has 8 x 32 rows of
+// outputs whatever the volume, so that very many small or flat volumes take a
+// pass an axis sooner (16384 x 2 volumes of 4^3 to 2^3, order 3: 0.23 ms fused,
+// 0.06 not), and so do double volumes above order 3, where a plane's 16
+// outputs a thread cost most (512 x 512 x 24 by 1.5: 0.69 and 0.36).  The
+// choice compares the two estimates, which were fitted to 1335 resizes (14
+// lattices, 13 factors, orders 0 to 7, both types), four in five within 15 %.
+// Of the 203 that the kernel would slow down by more than 5 % it leaves 13; of
+// 1068 on other lattices, 8 (at worst 0.27 -> 0.38 ms, 20000 volumes of 6^3
+// doubled, order 3).
+// False otherwise (the caller then runs a pass an axis).
 template <typename T>
 static bool rs_fused(const T *input, T *output, const RsArgs &a, hipStream_t st) {
   for (int d = 0; d < 3; ++d)
@@ -620,7 +664,8 @@ static bool rs_fused(const T *input, T *output, const RsArgs &a, hipStream_t st)
   const int txo = tall ? 16 : 4;
   const int ntx = (a.nt[0] + txo - 1) / txo;
   const long long nb = per * ntx;
-  if (!launch_fits(nb, RS_BLOCK)) return false;
+  const bool aligned = ((uintptr_t)input | (uintptr_t)output) % (4 * sizeof(T)) == 0;
+  if (!launch_fits(nb, RS_BLOCK) || rf_time<T>(a, wide, txo, nb) >= rs_passes_time<T>(a, aligned)) return false;
   const dim3 g((unsigned)nb), b(RS_BLOCK);
 #define RF_LAUNCH(TX, M) \
   hipLaunchKernelGGL((resize_fused<T, TX, M>), g, b, 0, st, input, output, a, ntx, nty, ntz, (unsigned)nb)
