@@ -148,13 +148,51 @@ struct GaOut {
   int tC;
 };
 
-template <int ORD, int MODE, bool ROLL, class TAPS>
+// Taps of NC channels at once, each multiplied by its target: their grid
+// gradients share the weights.
+template <int ORD, int NC, class TAPS>
+struct GaDot {
+  TAPS &t;
+  int sC;
+  float tv[NC];
+  __device__ __forceinline__ void row(const float *sp, int kx, int ky, float (&v)[ORD + 1]) const {
+    float u[NC][ORD + 1];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) t.row(sp + c * sC, kx, ky, u[c]);
+#pragma unroll
+    for (int k = 0; k <= ORD; ++k) {
+      v[k] = u[0][k] * tv[0];
+#pragma unroll
+      for (int c = 1; c < NC; ++c) v[k] += u[c][k] * tv[c];
+    }
+  }
+  __device__ __forceinline__ void next(int axis) { t.next(axis); }
+};
+
+// DOT: grid gradients take four channels at a time (sources whose channels
+// lie side by side: a cache line is read by few loads, not by one a channel).
+template <int ORD, int MODE, bool ROLL, bool DOT, class TAPS>
 __device__ __forceinline__ void ga_run(TAPS &taps, const float *src, int sC, int C, bool inb, bool valid,
                                        float (&w)[3][ORD + 1], float (&g)[3][ORD + 1], const GaOut &o,
                                        float (&og)[3]) {
   constexpr bool DERIV = TileMeta<MODE>::deriv;
+  int first = 0;
+  if constexpr (MODE == TM_GGRAD && DOT) {
 #pragma unroll 1
-  for (int c = 0; c < C; ++c) {
+    for (; first + 4 <= C; first += 4) {
+      if (!inb) continue;
+      GaDot<ORD, 4, TAPS> q{taps, sC, {}};
+#pragma unroll
+      for (int c = 0; c < 4; ++c) q.tv[c] = o.tp[(first + c) * o.tC];
+      float ax, ay, az;
+      ga_sum<ORD, DERIV, ROLL>(q, src + first * sC, w, g, ax, ay, az);
+      og[0] += ax;
+      og[1] += ay;
+      og[2] += az;
+    }
+  }
+#pragma unroll 1
+  for (int c = first; c < C; ++c) {
     float ax = 0.f, ay = 0.f, az = 0.f;
     if (inb) ga_sum<ORD, DERIV, ROLL>(taps, src + c * sC, w, g, ax, ay, az);
     if (!valid) continue;
@@ -174,7 +212,7 @@ __device__ __forceinline__ void ga_run(TAPS &taps, const float *src, int sC, int
   }
 }
 
-template <int ORD, int MODE, bool ZU, bool ROLL>
+template <int ORD, int MODE, bool ZU, bool ROLL, bool DOT = false>
 __device__ __forceinline__ void ga_sample(const PPArgs<float> &a, int n, int px, int py, int pz, bool valid) {
   constexpr int NT = ORD + 1;
   constexpr bool DERIV = TileMeta<MODE>::deriv;
@@ -213,7 +251,7 @@ __device__ __forceinline__ void ga_sample(const PPArgs<float> &a, int n, int px,
     t.s0 = st[0];
     t.s1 = st[1];
     t.s2 = st[2];
-    ga_run<ORD, MODE, ROLL>(t, src, sC, C, inb, valid, w, g, o, og);
+    ga_run<ORD, MODE, ROLL, DOT>(t, src, sC, C, inb, valid, w, g, o, og);
   } else {
     GaTaps<ORD, false, ZU, ROLL> t;
 #pragma unroll
@@ -226,7 +264,7 @@ __device__ __forceinline__ void ga_sample(const PPArgs<float> &a, int n, int px,
         t.ok[d] = ga_fold<ORD, DERIV>(a.bound[d], lo[d], sz[d], st[d], w[d], g[d], t.of[d]);
       }
     }
-    ga_run<ORD, MODE, ROLL>(t, src, sC, C, inb, valid, w, g, o, og);
+    ga_run<ORD, MODE, ROLL, DOT>(t, src, sC, C, inb, valid, w, g, o, og);
   }
   if constexpr (MODE == TM_GGRAD || MODE == TM_GGRAD1) {
     if (valid) {

@@ -274,9 +274,13 @@ __device__ __forceinline__ void gt_run(const PPArgs<float> &a, float *box, const
   }
 }
 
-template <int ORD, int MODE, bool ONE>
+// fb: list of the tiles left to the binned pass, or null: those whose box holds
+// more than 1 / parts of the LDS.  DIRECT (wide strided sources at order 1):
+// tiles that would stage one channel at a time (grid gradients: two) are read
+// from the caches instead.
+template <int ORD, int MODE, bool ONE, bool DIRECT>
 __global__ __launch_bounds__(256) void gtile_kernel(PPArgs<float> a, int ntx, int nty, int ntz,
-                                                                     int64_t nblocks, int *fb) {
+                                                    int64_t nblocks, int *fb, int parts) {
   using B = GTile<ORD, TileMeta<MODE>::deriv, ONE>;
   constexpr int NT = ORD + 1, R = B::R, STEP = B::NW;
   __shared__ __align__(16) float box[B::CAP];
@@ -367,15 +371,16 @@ __global__ __launch_bounds__(256) void gtile_kernel(PPArgs<float> a, int ntx, in
   fits = fits || none;
   int ncc = ONE ? 1 : a.C >= 3 ? 4 : (int)a.C;
   const int vol = d.e[0] * d.e[1] * d.e[2];
-  if (fb && (!fits || vol * 2 > B::CAP)) {   // listed for the binned pass
+  if (fb && (!fits || vol * parts > B::CAP)) {   // listed for the binned pass
     if (threadIdx.x == 0) fb[1 + atomicAdd(fb, 1)] = (int)tile;
     return;
   }
   while (ncc > 1 && vol * ncc > B::CAP) ncc >>= 1;
-  if (!fits || vol > B::CAP) {   // taps from the caches
+  constexpr int DIRECT_NCC = !DIRECT ? 0 : MODE == TM_GGRAD ? 2 : 1;
+  if (!fits || vol > B::CAP || ncc <= DIRECT_NCC) {   // taps from the caches
 #pragma unroll 1
     for (int py = s.py; py < s.py + R * STEP; py += STEP)
-      ga_sample<ORD, MODE, false, true>(a, s.n, s.px, py, s.pz, s.px < a.tX && py < a.tY && s.pz < a.tZ);
+      ga_sample<ORD, MODE, false, !DIRECT, DIRECT>(a, s.n, s.px, py, s.pz, s.px < a.tX && py < a.tY && s.pz < a.tZ);
     return;
   }
   d.DYZ = gt_plane<B::CAP>(d.e[0], d.e[1], d.e[2], ncc);
@@ -415,20 +420,26 @@ __global__ __launch_bounds__(256) void gtile_kernel(PPArgs<float> a, int ntx, in
   gt_run<ORD, MODE, 1>(a, box, d, fofs, fsg, s);
 }
 
+// Sources of many channels whose z neighbours are apart (channels-last views):
+// staging fewer than four channels at a time reads every cache line once for
+// each stage.
+static inline bool wide_strided(const PPArgs<float> &a) { return a.src_s[4] != 1 && a.C >= 8; }
+
 // fb: list of tiles left to the binned pass (a count, then tile ids), or null.
 template <int ORD, int MODE>
-static void launch_gtile(const PPArgs<float> &a, int *fb, hipStream_t st) {
+static void launch_gtile(const PPArgs<float> &a, int *fb, int parts, hipStream_t st) {
   using B = GTile<ORD, false, false>;
   const int ntx = (int)((a.tX + B::TX - 1) / B::TX);
   const int nty = (int)((a.tY + B::TY - 1) / B::TY);
   const int ntz = (int)((a.tZ + B::TZ - 1) / B::TZ);
   const int64_t nb = a.N * (int64_t)ntx * nty * ntz;
-  if (a.C == 1)
-    hipLaunchKernelGGL((gtile_kernel<ORD, MODE, true>), dim3((unsigned)nb), dim3(B::NTH), 0, st, a, ntx, nty, ntz, nb,
-                       fb);
+  const dim3 g((unsigned)nb), b(B::NTH);
+  if (ORD == 1 && wide_strided(a))
+    hipLaunchKernelGGL((gtile_kernel<ORD, MODE, false, ORD == 1>), g, b, 0, st, a, ntx, nty, ntz, nb, fb, parts);
+  else if (a.C == 1)
+    hipLaunchKernelGGL((gtile_kernel<ORD, MODE, true, false>), g, b, 0, st, a, ntx, nty, ntz, nb, fb, parts);
   else
-    hipLaunchKernelGGL((gtile_kernel<ORD, MODE, false>), dim3((unsigned)nb), dim3(B::NTH), 0, st, a, ntx, nty, ntz, nb,
-                       fb);
+    hipLaunchKernelGGL((gtile_kernel<ORD, MODE, false, false>), g, b, 0, st, a, ntx, nty, ntz, nb, fb, parts);
 }
 
 // Channels up to which a call's taps are read straight from the caches
@@ -439,10 +450,14 @@ static void launch_gtile(const PPArgs<float> &a, int *fb, hipStream_t st) {
 // 0.074 against 0.090 ms and 0.165 against 0.22 warped, of 8 channels 0.25
 // against 0.20; the spatial gradient, whose stores weigh more, changes over
 // earlier.  Above, the (ORD + 1)^2 rows of a tap box cost the caches more
-// than the tile (order 3, one channel, rotated: 0.22 against 0.13 ms).
+// than the tile (order 3, one channel, rotated: 0.22 against 0.13 ms).  Where
+// z neighbours are apart (channels-last views), neighbouring lanes and the taps
+// of a row share cache lines less, and one channel is the limit at order 1
+// (pull of 3: 0.12 against 0.09 ms near the identity, 0.21 and 0.10 rotated).
 template <int ORD, int MODE>
-constexpr int gather_channels() {
-  return ORD == 0 ? INT_MAX : ORD == 1 ? (MODE == TM_SGRAD ? 2 : 3) : 0;
+static int gather_channels(const PPArgs<float> &a) {
+  if (ORD != 1) return ORD == 0 ? INT_MAX : 0;
+  return a.src_s[4] != 1 ? 1 : MODE == TM_SGRAD ? 2 : 3;
 }
 
 }  // namespace ni_amd

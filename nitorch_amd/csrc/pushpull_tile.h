@@ -809,32 +809,41 @@ __global__ __launch_bounds__(DYN_NTH) void tile_dyn(PPArgs<float> a, int ntx, in
 namespace ni_amd {
 
 // Channels from which the tiles of a large pull or grid_grad that are too
-// spread for a box of two channels are sorted into bins instead of staging
-// one channel at a time: with fewer, or in small calls, the sort costs more
-// than it saves (order 3, 181 x 217 x 181, a warp of 8 voxels RMS: 8 channels
-// 1.2 ms binned, 2.6 not; one channel 0.58 and 0.38).
+// spread are sorted into bins instead of staging one or two channels at a
+// time: with fewer, or in small calls, the sort costs more than it saves (order
+// 3, 181 x 217 x 181, a warp of 8 voxels RMS: 8 channels 1.2 ms binned, 2.6
+// not; one channel 0.58 and 0.38).
 #define BIN_MIN_CHANNELS 3
+
+// Such a tile's box holds more than 1 / bin_parts of the LDS: two channels at a
+// time beat the bins (181 x 217 x 181, 4 channels, order 3, warp of 4 voxels
+// RMS: 0.50 against 0.57 ms), but not where each stage re-reads the source's
+// cache lines (16 channels last, order 3, rotation by 30 degrees: 2.68 and 1.56).
+template <int ORD, int MODE>
+static int bin_parts(const PPArgs<float> &a) {
+  return wide_strided(a) ? 4 : 2;
+}
 
 template <int ORD, int MODE>
 static void launch_gather_mode(const PPArgs<float> &a, hipStream_t st) {
-  if (a.C <= gather_channels<ORD, MODE>()) {
+  if (a.C <= gather_channels<ORD, MODE>(a)) {
     launch_gather<ORD, MODE>(a, st);
     return;
   }
-  if constexpr (ORD >= 2 && (MODE == TM_PULL || MODE == TM_SGRAD)) {
+  if constexpr (ORD >= 1 && (MODE == TM_PULL || MODE == TM_SGRAD)) {
     using B = TileDims<ORD, MODE>;
     const int ntx = (int)((a.tX + B::TX - 1) / B::TX);
     const int nty = (int)((a.tY + B::TY - 1) / B::TY);
     const int ntz = (int)((a.tZ + B::TZ - 1) / B::TZ);
     BinPlan p;
-    if (a.C >= BIN_MIN_CHANNELS && a.N * a.tX * a.tY * a.tZ >= BIN_MIN_SAMPLES &&
+    if ((ORD > 1 || wide_strided(a)) && a.C >= BIN_MIN_CHANNELS && a.N * a.tX * a.tY * a.tZ >= BIN_MIN_SAMPLES &&
         bin_plan(a, a.N * (int64_t)ntx * nty * ntz, B::TX * B::TY * B::TZ, p, st)) {
-      launch_gtile<ORD, MODE>(a, p.fb, st);
+      launch_gtile<ORD, MODE>(a, p.fb, bin_parts<ORD, MODE>(a), st);
       launch_binned<ORD, MODE>(a, ntx, nty, ntz, p, st);
       return;
     }
   }
-  if constexpr (ORD > 0) launch_gtile<ORD, MODE>(a, nullptr, st);
+  if constexpr (ORD > 0) launch_gtile<ORD, MODE>(a, nullptr, 0, st);
 }
 
 // Whether the mode's first kernel can cover the samples in one launch (thin or
@@ -842,7 +851,7 @@ static void launch_gather_mode(const PPArgs<float> &a, hipStream_t st) {
 template <int ORD, int MODE>
 static bool tile_fits(const PPArgs<float> &a) {
   using B = TileDims<ORD, MODE>;
-  const bool cache = TileMeta<MODE>::gather && a.C <= gather_channels<ORD, MODE>();
+  const bool cache = TileMeta<MODE>::gather && a.C <= gather_channels<ORD, MODE>(a);
   const int64_t bx = cache ? GA_TX : B::TX, by = cache ? GA_TY : B::TY, bz = cache ? GA_TZ : B::TZ;
   return launch_fits(a.N * ((a.tX + bx - 1) / bx) * ((a.tY + by - 1) / by) * ((a.tZ + bz - 1) / bz),
                      TileMeta<MODE>::gather ? GA_NTH : TileBox<ORD>::NTH);

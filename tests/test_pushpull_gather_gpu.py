@@ -81,3 +81,35 @@ def test_outside_taps_are_not_read(order, channels):
     out = G.grid_pull(T(x), T(g), ["zero"], [order], 1).cpu().numpy()
     ref = O.grid_pull(x.astype(np.float64), g.astype(np.float64), "zero", order, 1, oob_f32=True)
     assert np.isnan(ref).any() and np.array_equal(np.isnan(out), np.isnan(ref))
+
+
+@pytest.mark.parametrize("order", [1, 2, 3])
+@pytest.mark.parametrize("channels", [8, 9])
+def test_wide_channels_last_sources(order, channels):
+    """Sources of eight channels and more whose z stride is not 1: boxes that
+    would stage few channels at a time are read from the caches (order 1) or
+    sorted into bins (2^20 samples and more).  Small calls against the
+    oracle; large ones against the contiguous source."""
+    from nitorch_amd import grid as G
+    rng = np.random.default_rng(300 + 10 * order + channels)
+    for kind in ("near", "stretch", "scatter"):
+        shape, source = (5, 9, 33), (37, 23, 41)
+        g = grid(rng, shape, source, kind)
+        x = rng.standard_normal((1, channels) + source).astype(np.float32)
+        d = rng.standard_normal((1, channels) + shape).astype(np.float32)
+        g64, x64, d64 = (t.astype(np.float64) for t in (g, x, d))
+        xt = T(np.moveaxis(x, 1, -1)).movedim(-1, 1)
+        for bound, extrap in (("dct2", 0), ("zero", 1)):
+            case = (kind, order, channels, bound, extrap)
+            out = G.grid_pull(xt, T(g), [bound], [order], extrap)
+            check(out, O.grid_pull(x64, g64, bound, order, extrap, oob_f32=True), order, ("pull",) + case)
+            out = G.grid_grad(xt, T(g), [bound], [order], extrap)
+            check(out, O.grid_grad(x64, g64, bound, order, extrap, oob_f32=True), order, ("grad",) + case)
+            out, = G.grid_pull_backward(T(d), xt, T(g).requires_grad_(), [bound], [order], extrap)
+            ref = O.grid_pull_backward(d64, x64, g64, bound, order, extrap, oob_f32=True)[1]
+            check(out, ref, order, ("grid gradient",) + case)
+        g = grid(rng, (102, 101, 103), (102, 101, 103), kind)
+        x = torch.from_numpy(rng.standard_normal((1, 102, 101, 103, channels)).astype(np.float32)).cuda().movedim(-1, 1)
+        for fn in (G.grid_pull, G.grid_grad):
+            ref = fn(x.contiguous(), T(g), ["dct2"], [order], 0).cpu().double().numpy()
+            check(fn(x, T(g), ["dct2"], [order], 0), ref, order, (fn.__name__, kind))
