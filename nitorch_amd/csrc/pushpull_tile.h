@@ -815,13 +815,18 @@ namespace ni_amd {
 // not; one channel 0.58 and 0.38).
 #define BIN_MIN_CHANNELS 3
 
-// Such a tile's box holds more than 1 / bin_parts of the LDS: two channels at a
-// time beat the bins (181 x 217 x 181, 4 channels, order 3, warp of 4 voxels
-// RMS: 0.50 against 0.57 ms), but not where each stage re-reads the source's
-// cache lines (16 channels last, order 3, rotation by 30 degrees: 2.68 and 1.56).
+// Such a tile's box holds more than 1 / bin_parts of the LDS.  Two channels at
+// a time beat the bins up to order 4 (181 x 217 x 181, 4 channels, order 3, warp
+// of 4 voxels RMS: 0.50 against 0.57 ms), not where a sample has 216 taps or
+// more and the box most of a tile's time (order 5, warp of 8: 1.40 against 1.21;
+// of 2: 0.67 and 0.75, few tiles; order 4, 8 channels, warp of 8: 1.92 and 1.60),
+// but again at order 7, whose bins of 15^3 voxels are slow (rotation by 30
+// degrees: 1.57 and 1.96), nor where each stage re-reads the source's cache
+// lines (16 channels last, order 3, rotation by 30 degrees: 2.68 and 1.56).
 template <int ORD, int MODE>
 static int bin_parts(const PPArgs<float> &a) {
-  return wide_strided(a) ? 4 : 2;
+  const bool taps = MODE == TM_PULL && (ORD == 5 || ORD == 6 || (ORD == 4 && a.C > 4));
+  return taps || wide_strided(a) ? 4 : 2;
 }
 
 template <int ORD, int MODE>
