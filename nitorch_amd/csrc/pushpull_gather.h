@@ -245,7 +245,9 @@ __device__ __forceinline__ void ga_sample(const PPArgs<float> &a, int n, int px,
   if constexpr (MODE == TM_GGRAD)
     o.tp = a.trgt + (int)(n * a.trgt_s[0] + px * a.trgt_s[2] + py * a.trgt_s[3] + pz * a.trgt_s[4]);
   float og[3] = {0.f, 0.f, 0.f};
-  if (!ROLL && __all(inner[0] && inner[1] && inner[2])) {
+  if constexpr (ORD == 0 && (MODE == TM_GGRAD || MODE == TM_GGRAD1)) {
+    // zero everywhere: nothing to read
+  } else if (!ROLL && __all(inner[0] && inner[1] && inner[2])) {
     GaTaps<ORD, true, ZU, ROLL> t;
     t.base = lo[0] * st[0] + lo[1] * st[1] + lo[2] * st[2];
     t.s0 = st[0];

@@ -113,3 +113,15 @@ def test_wide_channels_last_sources(order, channels):
         for fn in (G.grid_pull, G.grid_grad):
             ref = fn(x.contiguous(), T(g), ["dct2"], [order], 0).cpu().double().numpy()
             check(fn(x, T(g), ["dct2"], [order], 0), ref, order, (fn.__name__, kind))
+
+
+@pytest.mark.parametrize("channels", [1, 3, 9])
+def test_nearest_grid_gradient_is_zero(channels):
+    """Whatever the source holds: nothing of it is read."""
+    from nitorch_amd import grid as G
+    rng = np.random.default_rng(channels)
+    shape = (5, 9, 17)
+    g = T(grid(rng, shape, shape, "near")).requires_grad_()
+    x = torch.full((1, channels) + shape, float("nan"), device="cuda")
+    out, = G.grid_pull_backward(torch.ones_like(x), x, g, ["dct2"], [0], 1)
+    assert out.shape == g.shape and not out.any()
