@@ -177,7 +177,9 @@ __device__ __forceinline__ void gt_sum(const typename GVec<NCC>::T *bp, const GB
           sv[c] += w[1][ky] * rg[c];
         }
       }
-      __builtin_amdgcn_sched_barrier(0);   // bound the rows in flight (registers)
+      // bound the rows in flight (registers; at order 2 the three rows of a plane
+      // fit, and the fence costs 2 to 5 %)
+      if constexpr (ORD != 2) __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
     for (int c = 0; c < NA; ++c) {
