@@ -34,6 +34,7 @@
 // splat3d :1235-1290, linear :1653-1858, nearest :2314-2341); folding and
 // signs follow bounds_common.h:28-219.
 #pragma once
+#include <algorithm>
 #include <climits>
 #include <type_traits>
 
@@ -829,6 +830,31 @@ static int bin_parts(const PPArgs<float> &a) {
   return taps || wide_strided(a) ? 4 : 2;
 }
 
+// A gather's samples are independent, and its blocks long along z: lattices of
+// few z are relabelled (points in a row and single slices to the last axes; two
+// or three slices trade z and y), so that their blocks are not mostly idle.
+// Pull, order 3: 10^6 points 0.90 -> 0.25 ms, 2048 x 2048 x 1 0.76 -> 0.23,
+// 1024 x 1024 x 2 0.21 -> 0.09.
+static PPArgs<float> gather_lattice(PPArgs<float> a) {
+  int64_t *t[3] = {&a.tX, &a.tY, &a.tZ};
+  auto swap = [&](int i, int j) {
+    std::swap(*t[i], *t[j]);
+    std::swap(a.grid_s[1 + i], a.grid_s[1 + j]);
+    std::swap(a.trgt_s[2 + i], a.trgt_s[2 + j]);
+    std::swap(a.out_s[2 + i], a.out_s[2 + j]);
+    std::swap(a.gout_s[1 + i], a.gout_s[1 + j]);
+  };
+  if (a.tZ == 1 && a.tY == 1) {
+    swap(0, 2);
+  } else if (a.tZ == 1) {   // (X, Y, 1) -> (1, X, Y)
+    swap(1, 2);
+    swap(0, 1);
+  } else if (a.tZ <= 3 && a.tY >= 16) {
+    swap(1, 2);
+  }
+  return a;
+}
+
 template <int ORD, int MODE>
 static void launch_gather_mode(const PPArgs<float> &a, hipStream_t st) {
   if (a.C <= gather_channels<ORD, MODE>(a)) {
@@ -854,7 +880,8 @@ static void launch_gather_mode(const PPArgs<float> &a, hipStream_t st) {
 // Whether the mode's first kernel can cover the samples in one launch (thin or
 // very many lattices leave most of a block idle, up to 255 of 256 threads).
 template <int ORD, int MODE>
-static bool tile_fits(const PPArgs<float> &a) {
+static bool tile_fits(const PPArgs<float> &call) {
+  const PPArgs<float> a = TileMeta<MODE>::gather ? gather_lattice(call) : call;
   using B = TileDims<ORD, MODE>;
   const bool cache = TileMeta<MODE>::gather && a.C <= gather_channels<ORD, MODE>(a);
   const int64_t bx = cache ? GA_TX : B::TX, by = cache ? GA_TY : B::TY, bz = cache ? GA_TZ : B::TZ;
@@ -871,7 +898,7 @@ static bool tile_fits(const PPArgs<float> &a) {
 template <int ORD, int MODE>
 static void launch_tile(const PPArgs<float> &a, hipStream_t st) {
   if constexpr (TileMeta<MODE>::gather) {
-    launch_gather_mode<ORD, MODE>(a, st);
+    launch_gather_mode<ORD, MODE>(gather_lattice(a), st);
   } else {
     using B = TileBox<ORD>;
     const int ntx = (int)((a.tX + B::TX - 1) / B::TX);

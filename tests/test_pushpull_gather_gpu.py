@@ -125,3 +125,30 @@ def test_nearest_grid_gradient_is_zero(channels):
     x = torch.full((1, channels) + shape, float("nan"), device="cuda")
     out, = G.grid_pull_backward(torch.ones_like(x), x, g, ["dct2"], [0], 1)
     assert out.shape == g.shape and not out.any()
+
+
+@pytest.mark.parametrize("shape", [(150, 1, 1), (1, 150, 1), (1, 1, 150), (33, 21, 1), (21, 33, 2), (9, 16, 3), (9, 15, 3),
+                                   (21, 1, 33)])
+@pytest.mark.parametrize("channels", [1, 4])
+def test_thin_lattices(shape, channels):
+    """Points, slices and a few slices, whose axes the gathers relabel."""
+    from nitorch_amd import grid as G
+    rng = np.random.default_rng(400 + channels)
+    source = (17, 23, 19)
+    x = rng.standard_normal((2, channels) + source).astype(np.float32)
+    d = rng.standard_normal((2, channels) + shape).astype(np.float32)
+    for kind in ("near", "scatter"):
+        g = np.concatenate([grid(rng, shape, source, kind) for _ in range(2)])
+        g64, x64, d64 = (t.astype(np.float64) for t in (g, x, d))
+        # the grid's components apart, the upstream channels last
+        gt = T(np.moveaxis(g, -1, 1)).movedim(1, -1)
+        dt = T(np.moveaxis(d, 1, -1)).movedim(-1, 1)
+        for order in (1, 2, 3):
+            case = (shape, channels, kind, order)
+            out = G.grid_pull(T(x), gt, ["dct2"], [order], 0)
+            check(out, O.grid_pull(x64, g64, "dct2", order, 0, oob_f32=True), order, ("pull",) + case)
+            out = G.grid_grad(T(x), gt, ["dct2"], [order], 0)
+            check(out, O.grid_grad(x64, g64, "dct2", order, 0, oob_f32=True), order, ("grad",) + case)
+            out, = G.grid_pull_backward(dt, T(x), gt.clone().requires_grad_(), ["dct2"], [order], 0)
+            ref = O.grid_pull_backward(d64, x64, g64, "dct2", order, 0, oob_f32=True)[1]
+            check(out, ref, order, ("grid gradient",) + case)
