@@ -125,8 +125,8 @@ def main():
     # the same pull / push on deformations far from the identity: the grid
     # recipe with the displacement rescaled to its nominal std (8 voxels RMS),
     # and an affine grid (15 degree rotation about y, zoom 1.1, about the
-    # centre); each with the fraction of tiles whose taps do not fit the LDS
-    # box (their samples are sorted by first-tap bin and run the binned pass)
+    # centre); each with the fraction of tiles that the tiles' own kernel
+    # leaves to a second pass (see fallback_fraction)
     deformed = {}
     for variant in ("rescaled", "affine"):
         if variant == "rescaled":
@@ -278,12 +278,16 @@ def affine_grid_192(dev, batch, angle_deg=15.0, zoom=1.1, shape=(192, 192, 192))
 
 
 def fallback_fraction(grid, shape, order, gather):
-    """Fraction of the tiles (4x8x16 samples for gathers, 8x16x16 for
-    scatters up to order 3) whose in-bound samples' first taps spread more
-    than the LDS box allows (tile extent + 1 per axis); those tiles' samples
-    are sorted by first-tap bin and run the binned second pass."""
+    """Fraction of the tiles with samples in bounds that the first kernel of a
+    multi-channel call leaves to a second pass, from the spread of their
+    samples' first taps.  Gathers (4 x 8 x 16 samples): the box of the tile's
+    taps holds more than half the LDS floats of a work-group, i.e. not two
+    channels (binned pass); orders 0 to 3 here.  Scatters (8 x 16 x 16 up to
+    order 5, 4 x 8 x 16 above): the taps spread more than the tile's extent +
+    order + 2 on an axis (larger boxes or binned pass)."""
     import torch
-    tile = (4, 8, 16) if (gather or order > 3) else (8, 16, 16)
+    tile = (4, 8, 16) if (gather or order > 5) else (8, 16, 16)
+    cap = 7592 if order <= 2 else 9824   # floats of a gather's box
     N = grid.shape[0]
     tol = 0.05
     lim = torch.tensor(shape, device=grid.device, dtype=grid.dtype) - 1 + tol
@@ -296,9 +300,7 @@ def fallback_fraction(grid, shape, order, gather):
         lo = torch.floor(grid - (order - 1) * 0.5)
     pad = [(-n) % t for n, t in zip(grid.shape[1:4], tile)]
     big = torch.tensor(2 ** 30, dtype=lo.dtype, device=lo.device)
-    fits = torch.ones((), dtype=torch.bool, device=grid.device)
-    nt = None
-    has = None
+    fits, volume, has = True, 1.0, None
     for d in range(3):
         v = lo[..., d]
         mn = torch.where(inb, v, big)
@@ -309,9 +311,12 @@ def fallback_fraction(grid, shape, order, gather):
         mn = mn.reshape(N, tx, tile[0], ty, tile[1], tz, tile[2]).amin((2, 4, 6))
         mx = mx.reshape(N, tx, tile[0], ty, tile[1], tz, tile[2]).amax((2, 4, 6))
         has = mn <= mx
-        fits = fits & (mx - mn <= tile[d] + 1)
-        nt = has.numel()
-    return round(float((has & ~fits).sum()) / nt, 4)
+        extent = mx - mn + order + 1
+        volume = volume * extent.double()
+        fits = fits & (extent <= (64 if gather else tile[d] + order + 2))
+    if gather:
+        fits = fits & (2 * volume <= cap)
+    return round(float((has & ~fits).sum()) / has.numel(), 4)
 
 
 def measured_traffic(op):

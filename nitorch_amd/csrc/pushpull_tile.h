@@ -47,9 +47,14 @@ namespace ni_amd {
 // Tiles whose bounding box holds at most ST_MAX_VOL elements (one or two boxes
 // of scatter_kernel) go to it, unless more than 1 / ST_FAR as many tiles are
 // wider: then all are binned -- a bin costs the same with few samples in it.
-// 181 x 217 x 181, order 3, one channel: rotation by 15 degrees and zoom 1.1
-// 546 us binned, 353 here; smooth warps of 2 / 4 / 6 voxels RMS 691 / 724 / 717
-// binned, 468 / 634 / 718 here; 8 channels, order 1, 6 voxels: 1263 and 1352.
+// 181 x 217 x 181, order 3, one channel, all binned against this rule: rotation
+// by 15 degrees and zoom 1.1 543 and 342 us; smooth warps of 2 / 4 / 6 / 8
+// voxels RMS 688 / 716 / 716 / 721 and 461 / 624 / 701 / 713.  Order 1, 8
+// channels: 963 and 876; 1111 / 1230 / 1263 / 1261 and 974 / 1140 / 1262 / 1256.
+// No call measured at orders 1 to 7 with 1 to 8 channels on these grids is
+// slower by more than 1 %; the one shape that is (2000 x 30 x 30 under a noise
+// of 0.3 voxels, order 3, 8 channels: 896 and 1034) leaves most work-groups
+// with one tile.
 #define ST_MAX_VOL 14000
 #define ST_FAR 8
 
@@ -527,15 +532,14 @@ __global__ __launch_bounds__((TileBox<ORD>::NTH),
   }
 }
 
-// Tiles whose box does not fit, by the direct per-sample routine.  With a
-// list (fb: count, then the tile ids that tile_kernel found too scattered)
-// a fixed grid walks the list; without one, every tile repeats tile_kernel's
-// bounding-box test (bit-identical, so every tile is handled by exactly one
-// of the two kernels).  Kept apart from tile_kernel so that its register
-// demand does not lower that kernel's occupancy.
+// Tiles whose box does not fit, by the direct per-sample routine, where no list
+// can be had: every tile repeats tile_kernel's bounding-box test (bit-identical,
+// so every tile is handled by exactly one of the two kernels).  Kept apart from
+// tile_kernel so that its register demand does not lower that kernel's
+// occupancy.
 template <int ORD, int MODE>
 __global__ __launch_bounds__((TileBox<ORD>::NTH)) void tile_fallback(PPArgs<float> a, int ntx, int nty, int ntz,
-                                                          int64_t nblocks, const int *fb) {
+                                                                     int64_t nblocks) {
   constexpr int NT = ORD + 1;
   constexpr int FL = TileFlags<MODE>::value;
   using B = TileBox<ORD>;
@@ -543,22 +547,6 @@ __global__ __launch_bounds__((TileBox<ORD>::NTH)) void tile_fallback(PPArgs<floa
   const int X = (int)a.tX, Y = (int)a.tY, Z = (int)a.tZ;
   int sx, sy, sz0;
   tl_thread<B>(sx, sy, sz0);
-  if (fb) {
-    const int cnt = fb[0];
-    for (int64_t j = blockIdx.x; j < cnt; j += gridDim.x) {
-      int64_t r = fb[1 + j];
-      const int tz = (int)(r % ntz); r /= ntz;
-      const int ty = (int)(r % nty); r /= nty;
-      const int tx = (int)(r % ntx);
-      const int n = (int)(r / ntx);
-      const int px = tx * B::TX + sx, py = ty * B::TY + sy, pz0 = tz * B::TZ + sz0;
-#pragma unroll 1
-      for (int i = 0; i < R; ++i)
-        if (px < X && py < Y && pz0 + i < Z)
-          pp_sample<float, int32_t, ORD, FL, true>(a, n, px, py, pz0 + i);
-    }
-    return;
-  }
   __shared__ int red[B::NW][6];
   int64_t r = xcd_block(nblocks);
   const int tz = (int)(r % ntz); r /= ntz;
@@ -932,7 +920,7 @@ static void launch_tile(const PPArgs<float> &a, hipStream_t st) {
       hipLaunchKernelGGL((tile_dyn<ORD, MODE>), dim3(gd), dim3(DYN_NTH), 0, st, a, ntx, nty, ntz, (const int *)fb);
       if (own) (void)hipFreeAsync(fb, st);
     } else {
-      hipLaunchKernelGGL((tile_fallback<ORD, MODE>), g, b, 0, st, a, ntx, nty, ntz, nb, (const int *)nullptr);
+      hipLaunchKernelGGL((tile_fallback<ORD, MODE>), g, b, 0, st, a, ntx, nty, ntz, nb);
     }
   }
 }

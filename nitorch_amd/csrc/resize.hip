@@ -463,7 +463,7 @@ static int rf_extent(const RsArgs &a, int d, int cnt) {
 
 template <typename T, int TXO, int MT>
 __global__ __launch_bounds__(RS_BLOCK) void resize_fused(const T *__restrict__ in, T *__restrict__ out, RsArgs a,
-                                                         int ntx, int nty, int ntz, unsigned nblocks) {
+                                                         int ntx, int nty, int ntz) {
   __shared__ T stage[RF_STAGE];
   __shared__ T tz[RF_OY * MT * RF_OZ];
   __shared__ T wx[TXO * MT * TXO];
@@ -668,7 +668,7 @@ static bool rs_fused(const T *input, T *output, const RsArgs &a, hipStream_t st)
   if (!launch_fits(nb, RS_BLOCK) || rf_time<T>(a, wide, txo, nb) >= rs_passes_time<T>(a, aligned)) return false;
   const dim3 g((unsigned)nb), b(RS_BLOCK);
 #define RF_LAUNCH(TX, M) \
-  hipLaunchKernelGGL((resize_fused<T, TX, M>), g, b, 0, st, input, output, a, ntx, nty, ntz, (unsigned)nb)
+  hipLaunchKernelGGL((resize_fused<T, TX, M>), g, b, 0, st, input, output, a, ntx, nty, ntz)
   if (tall) {
     if (wide) RF_LAUNCH(16, 8);
     else RF_LAUNCH(16, 4);
